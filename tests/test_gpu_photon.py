@@ -192,3 +192,25 @@ def test_shape_filtered_order_equals_the_reference_heap_order(rt, gpu_ctx, k, ra
         assert np.array_equal(got[2][i, :c], want[2][i, :c]), i
     assert np.all(got[0][qs == 45] == 0)
     assert (got[0] == k).mean() > 0.5
+
+
+@pytest.mark.parametrize("k", [1, 2, 3, 7, 8, 31, 63, 64, 100, 127, 128, 129])
+def test_long_searches_keep_the_reference_heap_order(rt, gpu_ctx, k):
+    """Queries between clusters visit thousands of nodes: the search gives
+    them up to whole wavefronts, which take subtrees of 64 photons at a time
+    (and, with 12,000 such queries, runs out of places for them).  Counts,
+    photons, distances and order must stay the reference's, at every heap
+    depth and with fewer queries than wavefronts."""
+    rng = np.random.default_rng(300 + k)
+    c = np.array([[0, 0, 0], [3, 0.2, 0.1], [1.4, 2.5, 0.3], [1.5, 1.2, 2.8]])
+    x = (c[rng.integers(0, 4, 40000)] + rng.normal(0, 0.1, (40000, 3))).astype(np.float32)
+    x = np.unique(x, axis=0)
+    tree = oracle.kd_build(x)[:2]
+    for nq, spread in ((3, 0.25), (1500, 0.25), (12000 if k in (8, 100) else 4000, 0.25), (3000, 1.0)):
+        print(f"[photon] long searches k={k} nq={nq} spread={spread}", flush=True)
+        q = (np.array([1.5, 0.9, 0.8]) + rng.normal(0, spread, (nq, 3))).astype(np.float32)
+        got = gpu_knn(rt, gpu_ctx, x, q, k, 100.0)
+        want = oracle.knn(x, q, k, 100.0, tree=tree)
+        assert np.array_equal(got[0], want[0])
+        assert np.array_equal(got[1], want[1])
+        assert np.array_equal(got[2], want[2])

@@ -212,3 +212,60 @@ def test_far_child_walk_with_signatures_equals_the_reference_search(coplanar):
             assert len(ids) == cnt[i]
             assert ids == idx[i, :cnt[i]].tolist(), (k, radius, i)
             assert np.array_equal(np.float32(ds), dist[i, :cnt[i]])
+
+
+@pytest.mark.parametrize("parked", [1, 4, 64])
+def test_parked_photons_leave_the_search_as_it_is(parked):
+    """The kernel walks on with an older radius while up to `parked` photons
+    wait for the heap, and makes the exact test when they reach it: the same
+    photons in the same order as the oracle, although more nodes are met."""
+    rng = np.random.default_rng(5 + parked)
+    c = rng.random((4, 3))
+    x = np.unique((c[rng.integers(0, 4, 2000)] + rng.normal(0, 0.05, (2000, 3))).astype(np.float32), axis=0)
+    order, axis, _ = oracle.kd_build(x)
+    nodes = x[order]
+    q = rng.random((60, 3)).astype(np.float32)
+    k, radius = 12, 100.0
+    cnt, idx, dist = oracle.knn(x, q, k, radius, tree=(order, axis))
+    for i in range(len(q)):
+        h, maxd, wait, stack = SlotHeap(k), np.float32(radius), [], []
+        l, r = 0, len(nodes)
+        while True:
+            done = False
+            if r <= l:
+                if stack:
+                    a, b, pd = stack.pop()
+                    if pd < maxd:
+                        l, r = a, b
+                else:
+                    done = True
+            if r > l:
+                med = l + (r - l) // 2
+                d = _norm(*(q[i] - nodes[med]))
+                diff = np.float32(q[i][axis[med]] - nodes[med][axis[med]]) if r - l > 1 else np.float32(0)
+                lo, hi = (l, med), (med + 1, r)
+                (l, r), far = (lo, hi) if diff < 0 else (hi, lo)
+                if far[1] > far[0]:
+                    stack.append((*far, abs(diff)))  # the root of a rounded square of one number is that number
+                if d < maxd:
+                    if h.cnt < k:
+                        h.take(d, int(order[med]))
+                    else:
+                        wait.append((d, int(order[med])))
+            if done or len(wait) >= parked:
+                for d, e in wait:
+                    if d < maxd:
+                        h.take(d, e)
+                        maxd = np.float32(h.D[0])
+                wait = []
+            if done:
+                break
+        ids, ds = h.result()
+        assert ids == idx[i, :cnt[i]].tolist()
+        assert np.array_equal(np.float32(ds), dist[i, :cnt[i]])
+
+
+def test_root_of_a_rounded_square():
+    rng = np.random.default_rng(1)
+    v = np.exp(rng.uniform(np.log(1e-18), np.log(1e18), 200000)).astype(np.float32)
+    assert np.array_equal(np.sqrt(v * v), v)
