@@ -19,6 +19,7 @@
 // moments and gradients are FP32.
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <cstdint>
 
 #include <hipcub/device/device_radix_sort.hpp>
@@ -440,14 +441,211 @@ __global__ __launch_bounds__(256) void k_fill(float *__restrict__ p, uint32_t co
     for (uint32_t i = blockIdx.x * 256 + threadIdx.x; i < count; i += gridDim.x * 256) p[i] = value;
 }
 
-// inference output: rgb = max(Y[:, 0..2], 0)
-__global__ __launch_bounds__(256) void k_out_rgb(const float *__restrict__ Y, uint32_t n,
-                                                 const uint32_t *__restrict__ n_dev, float *__restrict__ rgb)
+// ---------------------------------------------------------------------
+// Inference in one kernel: encoding and all five layers of a 16-row strip in
+// the registers of one wavefront.
+//
+// Each layer is computed transposed, Y^T = W^T X^T.  v_mfma_f32_16x16x16
+// returns D[m][n] with n = l % 16 and m = 4 (l / 16) + r in lane l, register
+// r, and takes B[k][n] with k = 4 (l / 16) + 0..3 from lane l: with n the row
+// and m (then k) the feature, a layer's result is the next layer's operand in
+// the same lane, and only ReLU and rounding to BF16 stand between them.  So
+// lane l holds features 16t + 4 (l / 16) + 0..3 of row l % 16: of the encoding
+// that is two grid levels per tile, and the four lanes of a row share its
+// 8 x levels gathers.
+//
+// What bounds it: the gathers.  A pair of corners one x apart lies in one
+// 8-byte word of a dense level, and of a hashed one when x is even, so a
+// level takes 4 loads, or 8 where x is odd, instead of 8.  One wavefront
+// needs 68 matrix instructions per strip; the weights (34 KB, in fragment
+// order) come through LDS and stay in registers (228 in all, two wavefronts per
+// SIMD; read from LDS for every strip, at five per SIMD, the kernel takes 432
+// to 480 us).  1,000,003 queries, 16 levels of 2^19 entries: 390 us, against
+// 1350 us in seven kernels per 65,536 rows with the activations in memory.  It
+// fetches about 70 cache lines of the hashed levels per row, 9 GB in all.
+// ---------------------------------------------------------------------
+constexpr uint32_t kXcds = 8;
+constexpr int kCacheFrags = 16 * 4 + 4;  // A fragments of W^T: four 64 x 64 layers, one 16 x 64
+
+typedef uint32_t u32x2u __attribute__((ext_vector_type(2), aligned(4)));
+typedef __bf16 bf2 __attribute__((ext_vector_type(2)));
+typedef float f32x2 __attribute__((ext_vector_type(2)));
+
+// Two floats rounded to nearest even, packed (the first in the low half).
+__device__ __forceinline__ uint32_t pack_bf16(float a, float b)
 {
-    if (n_dev) n = min(n, *n_dev);
-    for (uint32_t i = blockIdx.x * 256 + threadIdx.x; i < n; i += gridDim.x * 256)
+    const bf2 v = __builtin_convertvector((f32x2){a, b}, bf2);
+    return __builtin_bit_cast(uint32_t, v);
+}
+
+// Fragment f of W^T for lane l: out 16o + l % 16, inputs 16k + 4 (l / 16) + 0..3.
+__device__ __forceinline__ void load_weight_frags(const CacheDev &c, uint2 *frags)
+{
+    for (uint32_t e = threadIdx.x; e < kCacheFrags * 64; e += blockDim.x) {
+        const uint32_t f = e >> 6, l = e & 63u;
+        const uint32_t layer = f >> 4, o = f < 64 ? (f >> 2) & 3u : 0u, k = f & 3u;
+        frags[e] = *(const uint2 *)(c.w_t + kCacheLayerOffset(layer) + (16 * o + (l & 15u)) * kCacheWidth + 16 * k +
+                                    4 * (l >> 4));
+    }
+}
+
+// Trilinear features of grid level `lev` (resolution res) at p.
+__device__ __forceinline__ f32x2 grid_feature(const CacheDev &c, uint32_t lev, uint32_t res, bool dense, float px,
+                                              float py, float pz)
+{
+    const float r = (float)res;
+    const float x = px * r, y = py * r, z = pz * r;
+    const float fx0 = floorf(x), fy0 = floorf(y), fz0 = floorf(z);
+    const uint32_t x0 = (uint32_t)fx0, y0 = (uint32_t)fy0, z0 = (uint32_t)fz0;
+    const float fx = x - fx0, fy = y - fy0, fz = z - fz0;
+    const uint32_t x1 = min(x0 + 1, res), mask = c.table_size - 1u;
+    const uint32_t *tab = (const uint32_t *)c.grid_bf16 + (size_t)lev * c.table_size;
+    uint32_t i0[4], i1[4], at[4], v0[4], v1[4];
+    bool second = false;
 #pragma unroll
-        for (int c = 0; c < 3; ++c) rgb[(size_t)i * 3 + c] = fmaxf(Y[(size_t)i * 16 + c], 0.0f);
+    for (int k = 0; k < 4; ++k) {
+        const uint32_t yi = min(y0 + (k & 1), res), zi = min(z0 + (k >> 1), res);
+        if (dense) {
+            const uint32_t row = (res + 1) * (yi + (res + 1) * zi);
+            i0[k] = row + x0;
+            i1[k] = row + x1;
+            at[k] = min(i0[k], c.table_size - 2u);  // the pair stays inside the level
+        } else {
+            const uint32_t h = yi * 2654435761u ^ zi * 805459861u;
+            i0[k] = (x0 ^ h) & mask;
+            i1[k] = (x1 ^ h) & mask;
+            at[k] = i0[k] & ~1u;
+        }
+        second = second || i1[k] - at[k] > 1u;
+    }
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+        const u32x2u v = *(const u32x2u *)(tab + at[k]);
+        v0[k] = i0[k] == at[k] ? v.x : v.y;
+        v1[k] = i1[k] == at[k] ? v.x : v.y;
+    }
+    if (second) {
+#pragma unroll
+        for (int k = 0; k < 4; ++k) v1[k] = tab[i1[k]];
+    }
+    float f0 = 0, f1 = 0;
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+        const float wy = (k & 1) ? fy : 1 - fy, wz = (k >> 1) ? fz : 1 - fz;
+        const float w0 = (1 - fx) * wy * wz, w1 = fx * wy * wz;
+        f0 += w0 * bf2f((uint16_t)(v0[k] & 0xffffu));
+        f1 += w0 * bf2f((uint16_t)(v0[k] >> 16));
+        f0 += w1 * bf2f((uint16_t)(v1[k] & 0xffffu));
+        f1 += w1 * bf2f((uint16_t)(v1[k] >> 16));
+    }
+    return {f0, f1};
+}
+
+// The grid levels of a lane and their parameters: tile t, pair e is level
+// 8t + 2 (l / 16) + e.
+struct LaneLevels {
+    uint32_t res[4];
+    uint32_t dense;  // bit 2t + e
+};
+
+__device__ __forceinline__ LaneLevels lane_levels(const CacheDev &c, uint32_t q)
+{
+    LaneLevels ll{{1, 1, 1, 1}, 0};
+#pragma unroll
+    for (uint32_t i = 0; i < 4; ++i) {
+        const uint32_t lev = 8 * (i >> 1) + 2 * q + (i & 1u);
+        for (uint32_t l = 0; l < c.levels; ++l)
+            if (l == lev) {
+                ll.res[i] = c.res[l];
+                ll.dense |= (c.dense[l] ? 1u : 0u) << i;
+            }
+    }
+    return ll;
+}
+
+// The encoding of the strip's row l % 16: features 16t + 4 (l / 16) + 0..3 in x[t].
+__device__ __forceinline__ void encode_strip(const CacheDev &c, const LaneLevels &ll, const float *__restrict__ rec,
+                                             uint32_t q, bf16x4 x[4])
+{
+    float px, py, pz;
+    normalise_pos(c, rec, px, py, pz);
+    // feature 2 levels + j: normal, view direction, roughness, the constant 1, zeros
+    auto other = [&](uint32_t j) {
+        const float v = rec[3 + min(j, 6u)];
+        return j < 7u ? v : (j == 7u ? 1.0f : 0.0f);
+    };
+#pragma unroll
+    for (uint32_t t = 0; t < 4; ++t) {
+        uint32_t w[2];
+#pragma unroll
+        for (uint32_t e = 0; e < 2; ++e) {
+            const uint32_t lev = 8 * t + 2 * q + e;
+            f32x2 f;
+            if (t < 2 && lev < c.levels) {
+                const uint32_t i = 2 * (t & 1u) + e;
+                f = grid_feature(c, lev, ll.res[i], (ll.dense >> i) & 1u, px, py, pz);
+            } else {
+                const uint32_t j = 2 * (lev - c.levels);
+                f = {other(j), other(j + 1)};
+            }
+            w[e] = pack_bf16(f.x, f.y);
+        }
+        x[t] = __builtin_bit_cast(bf16x4, make_uint2(w[0], w[1]));
+    }
+}
+
+// One hidden layer in registers: x (features of a row) -> ReLU(W^T x).
+__device__ __forceinline__ void hidden_layer(const uint2 *frags, uint32_t layer, uint32_t lane, bf16x4 x[4])
+{
+    f32x4 acc[4];
+#pragma unroll
+    for (int o = 0; o < 4; ++o) {
+        acc[o] = f32x4{0, 0, 0, 0};
+#pragma unroll
+        for (int k = 0; k < 4; ++k)
+            acc[o] = mfma16(__builtin_bit_cast(bf16x4, frags[(layer * 16 + o * 4 + k) * 64 + lane]), x[k], acc[o]);
+    }
+#pragma unroll
+    for (int o = 0; o < 4; ++o)
+        x[o] = __builtin_bit_cast(bf16x4, make_uint2(pack_bf16(fmaxf(acc[o][0], 0.0f), fmaxf(acc[o][1], 0.0f)),
+                                                     pack_bf16(fmaxf(acc[o][2], 0.0f), fmaxf(acc[o][3], 0.0f))));
+}
+
+// The output layer: outputs 4 (l / 16) + r of row l % 16.
+__device__ __forceinline__ f32x4 output_layer(const uint2 *frags, uint32_t lane, const bf16x4 x[4])
+{
+    f32x4 y{0, 0, 0, 0};
+#pragma unroll
+    for (int k = 0; k < 4; ++k) y = mfma16(__builtin_bit_cast(bf16x4, frags[(64 + k) * 64 + lane]), x[k], y);
+    return y;
+}
+
+__global__ __launch_bounds__(256) void k_infer(CacheDev c, const float *__restrict__ in, uint32_t n,
+                                               const uint32_t *__restrict__ n_dev, float *__restrict__ rgb)
+{
+    __shared__ uint2 frags[kCacheFrags * 64];
+    if (n_dev) n = min(n, *n_dev);
+    // an eighth of the strips for each eighth of the blocks (see cache_infer)
+    const uint32_t strips = (n + 15) / 16, part = (strips + kXcds - 1) / kXcds;
+    const uint32_t lo = (blockIdx.x % kXcds) * part, hi = min(lo + part, strips);
+    if (lo + blockIdx.x / kXcds * 4 >= hi) return;  // whole block: before the barrier
+    load_weight_frags(c, frags);
+    __syncthreads();
+    const uint32_t lane = __lane_id(), wave = threadIdx.x / 64, q = lane >> 4;
+    const LaneLevels ll = lane_levels(c, q);
+    for (uint32_t s = lo + blockIdx.x / kXcds * 4 + wave; s < hi; s += gridDim.x / kXcds * 4) {
+        const uint32_t row = s * 16 + (lane & 15u);
+        bf16x4 x[4];
+        encode_strip(c, ll, in + (size_t)min(row, n - 1) * kCacheInStride, q, x);
+#pragma unroll
+        for (uint32_t l = 0; l + 1 < kCacheLayers; ++l) hidden_layer(frags, l, lane, x);
+        const f32x4 y = output_layer(frags, lane, x);
+        if (q == 0 && row < n) {
+            rgb[(size_t)row * 3] = fmaxf(y[0], 0.0f);
+            rgb[(size_t)row * 3 + 1] = fmaxf(y[1], 0.0f);
+            rgb[(size_t)row * 3 + 2] = fmaxf(y[2], 0.0f);
+        }
+    }
 }
 
 // ---------------------------------------------------------------------
@@ -476,12 +674,16 @@ hipError_t cache_forward(const CacheDev &c, const CacheWork &w, const float *in,
     return hipGetLastError();
 }
 
-hipError_t cache_infer(const CacheDev &c, const CacheWork &w, const float *in, uint32_t n, float *rgb, hipStream_t s,
+hipError_t cache_infer(const CacheDev &c, const float *in, uint32_t n, float *rgb, hipStream_t s,
                        const uint32_t *n_dev)
 {
-    hipError_t e = cache_forward(c, w, in, n, s, n_dev);
-    if (e != hipSuccess || n == 0) return e;
-    hipLaunchKernelGGL(k_out_rgb, grid_for(n, 256), dim3(256), 0, s, w.y, n, n_dev, rgb);
+    if (n == 0) return hipSuccess;
+    // Four wavefronts of 16 rows per block, two blocks per CU.  Blocks go to the
+    // eight XCDs in turn, and each XCD takes one contiguous eighth of the rows:
+    // rows in image order then touch an eighth of the grid's cells, which the
+    // XCD's own L2 holds.
+    const uint32_t blocks = std::min((n + 63) / 64, 512u);
+    hipLaunchKernelGGL(k_infer, dim3((blocks + kXcds - 1) / kXcds * kXcds), dim3(256), 0, s, c, in, n, n_dev, rgb);
     return hipGetLastError();
 }
 

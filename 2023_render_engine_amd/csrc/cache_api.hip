@@ -255,10 +255,7 @@ rt_status rt_cache_query(rt_cache *c, const float *in, uint32_t n, float *rgb, v
     std::lock_guard<std::recursive_mutex> g(rt::ctx_lock(c->ctx));
     RT_HIP(hipSetDevice(rt::ctx_device(c->ctx)));
     hipStream_t s = stream_ ? (hipStream_t)stream_ : (hipStream_t)rt::ctx_stream_ptr(c->ctx);
-    for (uint32_t i0 = 0; i0 < n; i0 += c->work.rows) {
-        const uint32_t m = std::min(c->work.rows, n - i0);
-        RT_HIP(rt::cache_infer(c->dev, c->work, in + (size_t)i0 * rt::kCacheInStride, m, rgb + (size_t)i0 * 3, s));
-    }
+    RT_HIP(rt::cache_infer(c->dev, in, n, rgb, s));
     return RT_OK;
 }
 

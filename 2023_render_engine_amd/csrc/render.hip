@@ -1138,14 +1138,13 @@ hipError_t chunk_iterate(const ChunkLaunch &c, const WaveParams &wp, uint32_t it
     // Training paths record there, trace kTrainSuffix more bounces and end
     // at the next cacheable vertex, whose cache answer completes their
     // target (self-training on the cache's own prediction).
-    const bool lookups = !B && wp.cache_depth != kNoCache && c.cache && c.cwork;
+    const bool lookups = !B && wp.cache_depth != kNoCache && c.cache;
     const bool photon = !B && c.photon != nullptr;
     if (photon && (lookups || wp.train || wp.harvest_shift != kNoHarvest)) return hipErrorInvalidValue;
     // a cache depth without lookups: only a plain wave that harvests records
     if (!wp.train && wp.cache_depth != kNoCache && !lookups && wp.harvest_shift == kNoHarvest)
         return hipErrorInvalidValue;
     if (B && wp.train) return hipErrorInvalidValue;
-    if (lookups && c.cwork->rows < c.capacity) return hipErrorInvalidValue;
     if (iterations & 1u) return hipErrorInvalidValue;
     const uint32_t ext_depth = !lookups ? kNoCache : (wp.train ? wp.cache_depth + kTrainSuffix : wp.cache_depth);
     const uint32_t need_record = wp.train ? 1u : 0u;
@@ -1204,7 +1203,7 @@ hipError_t chunk_iterate(const ChunkLaunch &c, const WaveParams &wp, uint32_t it
         if (lookups) {
             // cin rows are this iteration's queries (training records are
             // compacted into cin only by k_finalize, after this)
-            hipError_t e = cache_infer(*c.cache, *c.cwork, paths.cqin, c.capacity, paths.crgb, s,
+            hipError_t e = cache_infer(*c.cache, paths.cqin, c.capacity, paths.crgb, s,
                                        scount(q, kCCacheQ));
             if (e != hipSuccess) return e;
             hipLaunchKernelGGL(k_cache_apply, grid, blk, 0, s, paths, q);

@@ -59,8 +59,9 @@ size_t cache_sort_bytes(uint32_t rows);
 // fixed before the count is known.
 hipError_t cache_forward(const CacheDev &c, const CacheWork &w, const float *in, uint32_t n, hipStream_t s,
                          const uint32_t *n_dev = nullptr);
-hipError_t cache_infer(const CacheDev &c, const CacheWork &w, const float *in, uint32_t n, float *rgb,
-                       hipStream_t s, const uint32_t *n_dev = nullptr);
+// rgb = max(MLP(encoding(in)), 0) for any n; needs no scratch.
+hipError_t cache_infer(const CacheDev &c, const float *in, uint32_t n, float *rgb, hipStream_t s,
+                       const uint32_t *n_dev = nullptr);
 // Forward + loss + backward; accumulates gradients (c.grad, c.grid_grad) and
 // adds the summed loss to *loss (device, may be null).  With n_dev the row
 // count is min(n, *n_dev), read on the device.

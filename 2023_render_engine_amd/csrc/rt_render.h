@@ -275,7 +275,6 @@ struct ChunkLaunch {
     uint32_t capacity;
     float *res;                 // 3 floats per chunk path
     const CacheDev *cache;      // rendering with cache lookups (single scene)
-    const CacheWork *cwork;
     const BatchLaunch *batch;
     KernelProfile *prof;        // optional (never under graph capture)
     const PhotonLaunch *photon; // photon mapping (single scene, no cache)

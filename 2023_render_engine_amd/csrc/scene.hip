@@ -235,9 +235,6 @@ struct rt_scene {
     rt_render_stats stats{};
     rt::KernelProfile prof;  // event pairs of profiled frames (RT_FLAG_PROFILE)
     uint64_t stream_base = 0;
-    // radiance-cache inference scratch (one row per path slot), on demand
-    void *cache_arena = nullptr;
-    rt::CacheWork cwork{};
     // photon-mapping query rows (one per path slot), on demand
     void *photon_arena = nullptr;
     uint32_t photon_rows = 0;
@@ -283,9 +280,6 @@ rt_status ensure_result_buffer(WaveBuffers &w, uint64_t R, const char *who)
 static void free_arena(rt_scene *s)
 {
     free_wave_buffers(s->wb);
-    if (s->cache_arena) (void)hipFree(s->cache_arena);
-    s->cache_arena = nullptr;
-    s->cwork = rt::CacheWork{};
     if (s->photon_arena) (void)hipFree(s->photon_arena);
     s->photon_arena = nullptr;
     s->photon_rows = 0;
@@ -320,28 +314,6 @@ static rt_status ensure_photon_rows(rt_scene *s, uint32_t rows, PhotonLaunch &ph
     ph.qslot = (uint32_t *)(b + 3 * v3 + mat + u);
     ph.qrgb = (double *)(b + 3 * v3 + mat + 2 * u);
     ph.qbeta = (float *)(b + 3 * v3 + mat + 2 * u + rgb);
-    return RT_OK;
-}
-
-// Inference activations for `rows` cache queries (forward only).
-static rt_status ensure_cache_work(rt_scene *s, uint32_t rows)
-{
-    if (s->cache_arena && s->cwork.rows >= rows) return RT_OK;
-    if (s->cache_arena) (void)hipFree(s->cache_arena);
-    s->cache_arena = nullptr;
-    s->cwork = CacheWork{};
-    const size_t act = ((size_t)rows * kCacheWidth * 2 + 255) & ~(size_t)255;
-    const size_t y = (size_t)rows * kCacheOut * 4;
-    char *base = nullptr;
-    hipError_t e = hipMalloc(&base, act * kCacheLayers + y);
-    if (e != hipSuccess) {
-        set_error(std::string("rt_render_cached: cache scratch: ") + hipGetErrorString(e));
-        return e == hipErrorOutOfMemory ? RT_ERR_OOM : RT_ERR_HIP;
-    }
-    s->cache_arena = base;
-    s->cwork.rows = rows;
-    for (uint32_t l = 0; l < kCacheLayers; ++l) s->cwork.act[l] = (uint16_t *)(base + l * act);
-    s->cwork.y = (float *)(base + kCacheLayers * act);
     return RT_OK;
 }
 
@@ -880,10 +852,6 @@ static rt_status render_frames(const char *fn, rt_scene *s, const rt_render_opts
     rt_status st = rt::ensure_buffers(s, P, fn);
     if (st == RT_OK) st = rt::ensure_result_buffer(s->wb, R, fn);
     if (st != RT_OK) return st;
-    if (cache) {
-        st = rt::ensure_cache_work(s, s->wb.capacity);
-        if (st != RT_OK) return st;
-    }
     if (photon) {
         st = rt::ensure_photon_rows(s, s->wb.capacity, *photon);
         if (st != RT_OK) return st;
@@ -909,7 +877,6 @@ static rt_status render_frames(const char *fn, rt_scene *s, const rt_render_opts
     cl.capacity = std::min<uint32_t>(P, s->wb.capacity);
     cl.res = s->wb.res;
     cl.cache = cache ? &rt::cache_device(cache) : nullptr;
-    cl.cwork = cache ? &s->cwork : nullptr;
     cl.batch = nullptr;
     cl.prof = (flags & (RT_FLAG_PROFILE | RT_FLAG_COUNT)) ? &s->prof : nullptr;
     cl.photon = photon;
@@ -1039,7 +1006,6 @@ rt_status rt_cache_train_scene(rt_cache *c, rt_scene *s, const rt_render_opts *o
     hipStream_t stream = stream_ ? (hipStream_t)stream_ : (hipStream_t)rt::ctx_stream_ptr(s->ctx);
     const uint32_t P = rt::stripe_capacity(n_paths);
     rt_status st = rt::ensure_buffers(s, P, "rt_cache_train_scene");
-    if (st == RT_OK) st = rt::ensure_cache_work(s, s->wb.capacity);
     if (st != RT_OK) return st;
     RT_HIP(hipMemsetAsync(s->wb.queues.stats, 0, rt::kNumStats * 8, stream));
     rt::WaveParams wp{};
@@ -1061,7 +1027,6 @@ rt_status rt_cache_train_scene(rt_cache *c, rt_scene *s, const rt_render_opts *o
     cl.queues = s->wb.queues;
     cl.capacity = P;  // a slot for every training path: no read-back needed
     cl.cache = &rt::cache_device(c);  // training paths end in the cache after their suffix
-    cl.cwork = &s->cwork;
     // no host read-back: every training path starts at once and ends within max_depth iterations
     RT_HIP(rt::render_chunk(cl, film, wp, nullptr, stream));
     // the sample count stays on the device: no host round trip unless the

@@ -108,3 +108,29 @@ def test_online_training_fits_a_smooth_field(rt, gpu_ctx):
     t = field(rec)
     assert np.sqrt(np.mean((y - t) ** 2)) < 0.1
     cache.close()
+
+
+@pytest.mark.parametrize("levels,log2_table,base,scale", [(1, 8, 2, 1.0), (3, 9, 7, 1.7), (5, 12, 4, 2.0), (16, 10, 16, 1.38)])
+@pytest.mark.parametrize("n", [1, 15, 16, 17, 63, 64, 65, 1000, 70001])
+def test_query_sizes_and_level_counts(rt, gpu_ctx, orc, levels, log2_table, base, scale, n):
+    """Strips of 16 rows with remainders, level counts that end inside a
+    feature tile, dense levels that fill their table (res 7 and 512 entries),
+    positions on the box's faces (the last cell's clamped corners)."""
+    cache = rt.RadianceCache(gpu_ctx, (0, 0, 0), (1, 1, 1), levels=levels, log2_table=log2_table, base_res=base,
+                             per_level_scale=scale, batch=256, seed=3)
+    cfg = orc.cache_cfg(levels, log2_table, base, scale, (0, 0, 0), (1, 1, 1))
+    mlp, grid = cache.get_params()
+    grid = np.random.default_rng(11).uniform(-0.5, 0.5, grid.shape).astype(np.float32)
+    cache.set_params(mlp, grid)
+    rec = records(n, 1)
+    rec[:: 7, 0] = 1.0
+    rec[3:: 7, 1] = 0.0
+    rec[5:: 7, 2] = 1.0
+    y = cache.query(torch.from_numpy(rec).cuda()).cpu().numpy()
+    m = min(n, 2000)
+    at = np.r_[:m // 2, n - (m - m // 2):n]
+    ref = orc.cache_loss_grad(cfg, mlp, grid, rec[at], np.zeros((m, 3), np.float32), emulate_bf16=True,
+                              want_grad=False)[3]
+    ref = np.maximum(ref, 0)
+    assert np.max(np.abs(y[at] - ref)) <= 1e-2 * max(1.0, np.max(np.abs(ref)))
+    cache.close()
