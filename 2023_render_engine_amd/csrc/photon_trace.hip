@@ -111,6 +111,7 @@ __global__ __launch_bounds__(kPhBlock) void k_photon_trace(SceneDev sc, PhotonTr
     extern __shared__ int32_t s_stack[];
     StackTail<PathStack> s_tail;
     const PathStack stack{s_stack + threadIdx.x, s_tail};
+    stack_init(stack);
     const float4 *nodes = (const float4 *)sc.bvh.nodes;
     const float4 *tris = (const float4 *)sc.bvh.tris;
     uint32_t n_node = 0, n_tri = 0;
@@ -131,7 +132,7 @@ __global__ __launch_bounds__(kPhBlock) void k_photon_trace(SceneDev sc, PhotonTr
             TravState s;
             trav_begin(s, o.x, o.y, o.z, d.x, d.y, d.z, INFINITY, false, 0);
             if (sc.bvh.nodes)
-                while (!trav_step_any<WIDE, false, false>(s, nodes, tris, stack, cap, n_node, n_tri)) {
+                while (!trav_step_any<WIDE, false, false>(s, nodes, tris, stack, cap, kLeafBatch, n_node, n_tri)) {
                 }
             int32_t hid = s.hit;
             float th = s.thit;

@@ -28,6 +28,8 @@
 // Path slots, queues and their counters are striped (rt_render.h): a
 // workgroup serves stripe blockIdx % kStripes, so the appends of the whole
 // chip spread over 64 counters instead of queueing on one address.
+#include <algorithm>
+
 #include "rt_device.h"
 #include "rt_render.h"
 #include "rt_shade.h"
@@ -352,6 +354,7 @@ __global__ __launch_bounds__(kBlock) void k_extend(SceneDev sc0, BatchDev bt, Pa
     extern __shared__ int32_t s_stack[];
     StackTail<PathStack> s_tail;
     const PathStack stack{s_stack + threadIdx.x, s_tail};
+    stack_init(stack);
     const uint32_t *active = q.active[cur];
     const uint32_t cs = q.cs;
     auto count = [&](uint32_t j) { return *lcount(q, kLActive0 + cur, j); };
@@ -379,7 +382,7 @@ __global__ __launch_bounds__(kBlock) void k_extend(SceneDev sc0, BatchDev bt, Pa
             if (cursor_finished(c)) break;
             continue;
         }
-        if (has && trav_step_any<WIDE, false, STATS>(s, nodes, tris, stack, cap, n_node, n_tri)) {
+        if (has && trav_step_any<WIDE, false, STATS>(s, nodes, tris, stack, cap, leaf_batch(c), n_node, n_tri)) {
             ((float2 *)(path_rec(p, slot) + kPqHit))[1] = make_float2(s.thit, as_f(s.hit));
             has = false;
         }
@@ -888,6 +891,7 @@ __global__ __launch_bounds__(kBlock) void k_connect(SceneDev sc0, BatchDev bt, P
     extern __shared__ int32_t s_stack[];
     StackTail<PathStack> s_tail;
     const PathStack stack{s_stack + threadIdx.x, s_tail};
+    stack_init(stack);
     const size_t sstride = (size_t)q.cs * p.nee_stride;  // shadow rays per stripe
     auto count = [&](uint32_t j) { return *lcount(q, kLShadow, j); };
     StripeCursor c;
@@ -911,7 +915,7 @@ __global__ __launch_bounds__(kBlock) void k_connect(SceneDev sc0, BatchDev bt, P
             if (cursor_finished(c)) break;
             continue;
         }
-        if (has && trav_step_any<WIDE, true, STATS>(s, nodes, tris, stack, cap, n_node, n_tri)) {
+        if (has && trav_step_any<WIDE, true, STATS>(s, nodes, tris, stack, cap, leaf_batch(c), n_node, n_tri)) {
             if (s.occ) atomicAnd(path_word(p, sl >> 5, kPqRng, 3), ~(1u << (sl & 31u)));
             if (STATS) n_occ += s.occ ? 1u : 0u;
             has = false;
@@ -1070,8 +1074,9 @@ size_t extend_lds_bytes(uint32_t stack_cap)
 }
 
 // Workgroups of a persistent traversal launch: as many as fit on the chip
-// (LDS-limited, at most 16 per CU).
-static dim3 persistent_grid(size_t lds)
+// (LDS-limited, at most 16 per CU), and no more than `items` can occupy at
+// kMinWidth per wavefront.
+static dim3 persistent_grid(size_t lds, uint64_t items)
 {
     static int cus = 0;
     if (cus == 0) {
@@ -1082,7 +1087,8 @@ static dim3 persistent_grid(size_t lds)
     }
     size_t per_cu = lds ? (160u * 1024u) / lds : 16;
     per_cu = per_cu > 16 ? 16 : (per_cu < 1 ? 1 : per_cu);
-    return dim3((unsigned)(cus * per_cu));
+    const uint64_t need = (items + 2 * kMinWidth - 1) / (2 * kMinWidth);
+    return dim3((unsigned)std::max<uint64_t>(kStripes, std::min<uint64_t>((uint64_t)cus * per_cu, need)));
 }
 
 // Workgroups of the queue kernels: every stripe needs at least one.
@@ -1128,7 +1134,8 @@ hipError_t chunk_iterate(const ChunkLaunch &c, const WaveParams &wp, uint32_t it
     const size_t lds = extend_lds_bytes(stack_cap);
     const dim3 blk(kBlock);
     const dim3 grid = queue_grid(wp);
-    const dim3 pgrid = persistent_grid(lds);
+    const dim3 egrid = persistent_grid(lds, c.capacity);
+    const dim3 cgrid = persistent_grid(lds, (uint64_t)c.capacity * std::max(1u, c.paths.nee_stride));
     const PathsDev &paths = c.paths;
     const ShadowDev &shadow = c.shadow;
     QueuesDev q;
@@ -1159,14 +1166,14 @@ hipError_t chunk_iterate(const ChunkLaunch &c, const WaveParams &wp, uint32_t it
         if (ev) (void)hipEventRecord(e1, s);
     };
     auto extend = [&]() {
-        auto go = [&](auto kern) { hipLaunchKernelGGL(kern, pgrid, blk, lds, s, sc, bt, paths, q, cur, cap); };
+        auto go = [&](auto kern) { hipLaunchKernelGGL(kern, egrid, blk, lds, s, sc, bt, paths, q, cur, cap); };
         if (B && wide) cnt ? go(k_extend<true, true, true>) : go(k_extend<true, true, false>);
         else if (B) cnt ? go(k_extend<true, false, true>) : go(k_extend<true, false, false>);
         else if (wide) cnt ? go(k_extend<false, true, true>) : go(k_extend<false, true, false>);
         else cnt ? go(k_extend<false, false, true>) : go(k_extend<false, false, false>);
     };
     auto connect = [&]() {
-        auto go = [&](auto kern) { hipLaunchKernelGGL(kern, pgrid, blk, lds, s, sc, bt, paths, shadow, q, cap); };
+        auto go = [&](auto kern) { hipLaunchKernelGGL(kern, cgrid, blk, lds, s, sc, bt, paths, shadow, q, cap); };
         if (B && wide) cnt ? go(k_connect<true, true, true>) : go(k_connect<true, true, false>);
         else if (B) cnt ? go(k_connect<true, false, true>) : go(k_connect<true, false, false>);
         else if (wide) cnt ? go(k_connect<false, true, true>) : go(k_connect<false, true, false>);

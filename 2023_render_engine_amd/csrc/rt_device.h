@@ -132,8 +132,10 @@ __device__ __forceinline__ bool tri_intersects(const TriRay &r, const float4 a, 
     return true;
 }
 
-// Slab-test constants.  A zero direction component is replaced by +-1e-30
-// so no 0 * inf NaN can arise; the padded boxes keep the test conservative.
+// Slab-test constants.  A direction component below 1e-22 is replaced by
+// +-1e-22, so no 0 * inf NaN can arise and a node's scale times 2^24 / d stays
+// finite (scales up to 10^9); the padded boxes keep the test conservative.
+constexpr float kMinDir = 1e-22f;
 struct BoxRay {
     float ix, iy, iz;     // 1 / d
     float oix, oiy, oiz;  // o / d
@@ -142,9 +144,9 @@ struct BoxRay {
 __device__ __forceinline__ BoxRay make_box_ray(float ox, float oy, float oz, float dx, float dy, float dz)
 {
     BoxRay b;
-    float ddx = fabsf(dx) > 1e-30f ? dx : copysignf(1e-30f, dx);
-    float ddy = fabsf(dy) > 1e-30f ? dy : copysignf(1e-30f, dy);
-    float ddz = fabsf(dz) > 1e-30f ? dz : copysignf(1e-30f, dz);
+    float ddx = fabsf(dx) > kMinDir ? dx : copysignf(kMinDir, dx);
+    float ddy = fabsf(dy) > kMinDir ? dy : copysignf(kMinDir, dy);
+    float ddz = fabsf(dz) > kMinDir ? dz : copysignf(kMinDir, dz);
     b.ix = 1.0f / ddx; b.iy = 1.0f / ddy; b.iz = 1.0f / ddz;
     b.oix = ox * b.ix; b.oiy = oy * b.iy; b.oiz = oz * b.iz;
     return b;
@@ -191,14 +193,8 @@ constexpr int kTravBlock = 128;
 #ifndef RT_CLAIM_MIN
 #define RT_CLAIM_MIN 64
 #endif
-#ifndef RT_LEAF_BATCH
-#define RT_LEAF_BATCH 16
-#endif
 #ifndef RT_NODE_STEPS
 #define RT_NODE_STEPS 4
-#endif
-#ifndef RT_LEAF_BATCH_ANY
-#define RT_LEAF_BATCH_ANY 16
 #endif
 constexpr uint32_t kRefillLanes = RT_REFILL_LANES;  // refill a wavefront when at least this many lanes are idle
 
@@ -223,7 +219,8 @@ template <int L>
 struct TravStack {
     static_assert(L > 0 && L <= kMaxStack, "the LDS part holds 1..kMaxStack entries");
     static constexpr int kLds = L;
-    static constexpr int kTail = kMaxStack - L;  // private entries
+    // private entries (with the bottom mark and the place past the last entry)
+    static constexpr int kTail = L < kMaxStack ? kMaxStack + 2 - L : 0;
     int32_t *lds;   // this lane's column of the workgroup's LDS stack
     int32_t *tail;  // this lane's private overflow entries (kTail of them)
 };
@@ -258,13 +255,26 @@ __device__ __forceinline__ int32_t stack_get(const S &st, int sp)
 template <class S>
 inline size_t stack_lds_bytes(uint32_t stack_cap, uint32_t block)
 {
-    const uint32_t lds = stack_cap < (uint32_t)S::kLds ? stack_cap : (uint32_t)S::kLds;
+    // one entry more than the four-wide walk's pending ones (stack_cap - 1 of
+    // them): the mark at the bottom and the place past the last entry
+    const uint32_t need = stack_cap + 1;
+    const uint32_t lds = S::kTail == 0 || need < (uint32_t)S::kLds ? need : (uint32_t)S::kLds;
     return (size_t)lds * block * sizeof(int32_t);
 }
+
+// Entry 0 of a stack is kNoRef (stack_init, once per lane): popped when
+// nothing is left.
+constexpr int kStackBase = 1;
 
 // No node or leaf: a reference that no tree produces (a leaf reference is
 // ~(first << 3 | count - 1) with first + count <= 2^28).
 constexpr int32_t kNoRef = INT32_MIN;
+
+template <class S>
+__device__ __forceinline__ void stack_init(const S &st)
+{
+    st.lds[0] = kNoRef;
+}
 
 struct TravState {
     TriRay tr;
@@ -291,7 +301,7 @@ __device__ __forceinline__ void trav_begin(TravState &s, float ox, float oy, flo
     s.hit = -1;
     s.cur = root;
     s.leaf = kNoRef;
-    s.sp = 0;
+    s.sp = kStackBase;
     s.occ = false;
 }
 
@@ -315,7 +325,7 @@ __device__ __forceinline__ bool trav_step(TravState &s, const float4 *__restrict
         const int32_t c0 = __float_as_int(d.x), c1 = __float_as_int(d.y);
         if (h0 && h1) {
             const bool swap = t1 < t0;
-            if (s.sp < cap) {
+            if (s.sp < cap + kStackBase) {
                 stack_put(stack, s.sp, swap ? c0 : c1);
                 ++s.sp;
             }
@@ -344,7 +354,7 @@ __device__ __forceinline__ bool trav_step(TravState &s, const float4 *__restrict
             }
         }
     }
-    if (s.sp > 0) {
+    if (s.sp > kStackBase) {
         --s.sp;
         s.cur = stack_get(stack, s.sp);
         return false;
@@ -352,6 +362,12 @@ __device__ __forceinline__ bool trav_step(TravState &s, const float4 *__restrict
     return true;
 }
 
+// What bounds it (16M rays, 1M triangles): the L1's address and data path is
+// busy all the time (four 16-byte loads per visit, 33 lanes of 64 active) and
+// the vector units 81 % of it.  A visit is 125 vector instructions and no
+// branch: with conversions, and branches around each push, it was 135 and ten
+// branches, and the launch took 5.03 ms instead of 4.82.
+//
 // One step over the four-wide quantized tree (Node4, rt_internal.h): the
 // four child boxes are dequantized with one FMA per bound against the
 // node's origin and power-of-two scale, hit children are sorted by entry
@@ -370,21 +386,60 @@ __device__ __forceinline__ void cswap_key(uint32_t &ka, int32_t &ra, uint32_t &k
 
 // Leaves are not intersected the moment a lane reaches one: the lane parks
 // the leaf and keeps walking interior nodes, and the wavefront intersects
-// parked leaves together once kLeafBatch lanes hold one, or as soon as some
+// parked leaves together once a quarter of its lanes hold one, or as soon as some
 // lane cannot go on without it (a second leaf reached, or no nodes left).
 // Leaf work (up to four triangle tests) then runs with most lanes active
 // instead of one or two lanes holding the other 62 at every step.  Closest
 // hits are unchanged (the nearest accepted triangle does not depend on the
 // order of the tests, only ties would); culling against the running hit
 // distance starts a little later, so a ray may visit a few more nodes.
-constexpr uint32_t kLeafBatch = RT_LEAF_BATCH;        // closest hit
-constexpr uint32_t kLeafBatchAny = RT_LEAF_BATCH_ANY;  // any hit (shadow rays end at their first occluder)
+constexpr uint32_t kLeafBatch = 16;                   // of a full wavefront
 constexpr uint32_t kNodeSteps = RT_NODE_STEPS;         // interior-node visits per traversal step
+
+// The four bytes of w as two words of two halves: bits 0x00qq read as a half
+// are the number q 2^-24 exactly, which v_fma_mix_f32 takes as its first
+// factor, so a plane distance costs one FMA (against a scale 2^24 larger) and
+// half a mask instead of a conversion and an FMA, with the same rounding.
+constexpr uint32_t kTwo24 = 24u << 23;  // added to a float's bits: times 2^24
+struct BytePairs {
+    uint32_t even, odd;  // bytes 0 | 2 and 1 | 3
+};
+__device__ __forceinline__ BytePairs byte_pairs(uint32_t w)
+{
+    return {w & 0x00ff00ffu, __builtin_amdgcn_perm(w, 0u, 0x0c070c05u)};
+}
+__device__ __forceinline__ float byte_half(const BytePairs &b, int i)
+{
+    const uint32_t w = (i & 1) ? b.odd : b.even;
+    return (float)__builtin_bit_cast(_Float16, (unsigned short)(i >= 2 ? w >> 16 : w));
+}
+
+// Pushes ref[3], ref[2], ref[1] where their key is a hit.  Every entry is
+// written at the stack's end and counted or not, so the write past the last
+// entry needs a place: the stack holds one more than the tree can need.
+template <class S>
+__device__ __forceinline__ void stack_push3(const S &st, int &sp, const int32_t ref[4], const uint32_t key[4])
+{
+    if (S::kTail > 0 && __ballot(sp + 2 >= S::kLds) != 0) {
+#pragma unroll
+        for (int i = 3; i >= 1; --i)
+            if (key[i] != 0xffffffffu) {
+                stack_put(st, sp, ref[i]);
+                ++sp;
+            }
+        return;
+    }
+#pragma unroll
+    for (int i = 3; i >= 1; --i) {
+        st.lds[sp * kTravBlock] = ref[i];
+        sp += key[i] != 0xffffffffu ? 1 : 0;
+    }
+}
 
 template <bool ANY, bool STATS, class Stack, bool OPAQUE = false>
 __device__ __forceinline__ bool trav_step4(TravState &s, const float4 *__restrict__ nodes,
                                            const float4 *__restrict__ tris, const Stack &stack, int cap,
-                                           uint32_t &n_node, uint32_t &n_tri)
+                                           uint32_t leaf_batch, uint32_t &n_node, uint32_t &n_tri)
 {
     // kNodeSteps interior-node visits (each followed by parking a reached
     // leaf) per step, so the per-step refill and leaf-phase checks are paid
@@ -395,11 +450,13 @@ __device__ __forceinline__ bool trav_step4(TravState &s, const float4 *__restric
             if (STATS) ++n_node;
             const float4 *np = nodes + 4 * (size_t)s.cur;
             const float4 a = np[0], b = np[1], c = np[2], d = np[3];
+            const int32_t below = stack_get(stack, s.sp - 1);  // the next entry, should no child be hit
             const float tlim = ANY ? s.tmax * kHitScale : fminf(s.h, s.tmax) * kHitScale;
             const uint32_t meta = __float_as_uint(a.w);
-            const float Ax = __uint_as_float((meta & 0xffu) << 23) * s.br.ix;
-            const float Ay = __uint_as_float(((meta >> 8) & 0xffu) << 23) * s.br.iy;
-            const float Az = __uint_as_float(((meta >> 16) & 0xffu) << 23) * s.br.iz;
+            // the node's scales times 2^24 (byte_half) over the direction
+            const float Ax = __uint_as_float(((meta & 0xffu) << 23) + kTwo24) * s.br.ix;
+            const float Ay = __uint_as_float((((meta >> 8) & 0xffu) << 23) + kTwo24) * s.br.iy;
+            const float Az = __uint_as_float((((meta >> 16) & 0xffu) << 23) + kTwo24) * s.br.iz;
             const float Bx = fmaf(a.x, s.br.ix, -s.br.oix);
             const float By = fmaf(a.y, s.br.iy, -s.br.oiy);
             const float Bz = fmaf(a.z, s.br.iz, -s.br.oiz);
@@ -415,15 +472,13 @@ __device__ __forceinline__ bool trav_step4(TravState &s, const float4 *__restric
             const uint32_t qnz = nz ? qhz : qlz, qfz = nz ? qlz : qhz;
             uint32_t key[4];
             int32_t ref[4] = {__float_as_int(b.x), __float_as_int(b.y), __float_as_int(b.z), __float_as_int(b.w)};
+            const BytePairs nx2 = byte_pairs(qnx), fx2 = byte_pairs(qfx), ny2 = byte_pairs(qny), fy2 = byte_pairs(qfy),
+                            nz2 = byte_pairs(qnz), fz2 = byte_pairs(qfz);
     #pragma unroll
             for (int i = 0; i < 4; ++i) {
-                const int sh = 8 * i;
-                const float txn = fmaf((float)((qnx >> sh) & 0xffu), Ax, Bx);
-                const float txf = fmaf((float)((qfx >> sh) & 0xffu), Ax, Bx);
-                const float tyn = fmaf((float)((qny >> sh) & 0xffu), Ay, By);
-                const float tyf = fmaf((float)((qfy >> sh) & 0xffu), Ay, By);
-                const float tzn = fmaf((float)((qnz >> sh) & 0xffu), Az, Bz);
-                const float tzf = fmaf((float)((qfz >> sh) & 0xffu), Az, Bz);
+                const float txn = fmaf(byte_half(nx2, i), Ax, Bx), txf = fmaf(byte_half(fx2, i), Ax, Bx);
+                const float tyn = fmaf(byte_half(ny2, i), Ay, By), tyf = fmaf(byte_half(fy2, i), Ay, By);
+                const float tzn = fmaf(byte_half(nz2, i), Az, Bz), tzf = fmaf(byte_half(fz2, i), Az, Bz);
                 const float tn = fmaxf(fmaxf(txn, tyn), fmaxf(tzn, 0.0f));
                 float tf = fminf(fminf(txf, tyf), tzf);
                 tf = fminf(tf * kTfarScale, tlim);
@@ -437,36 +492,24 @@ __device__ __forceinline__ bool trav_step4(TravState &s, const float4 *__restric
                 cswap_key(key[1], ref[1], key[3], ref[3]);
                 cswap_key(key[1], ref[1], key[2], ref[2]);
             }
-            if (key[0] != 0xffffffffu) {
-    #pragma unroll
-                for (int i = 3; i >= 1; --i)
-                    if (key[i] != 0xffffffffu && s.sp < cap) {
-                        stack_put(stack, s.sp, ref[i]);
-                        ++s.sp;
-                    }
-                s.cur = ref[0];
-            } else if (s.sp > 0) {
-                --s.sp;
-                s.cur = stack_get(stack, s.sp);
-            } else {
-                s.cur = kNoRef;
-            }
+            // the far hits go onto the stack without a branch: each is written and
+            // the next overwrites it unless it counts
+            const bool any = key[0] != 0xffffffffu;
+            stack_push3(stack, s.sp, ref, key);
+            s.cur = any ? ref[0] : below;
+            s.sp -= any ? 0 : 1;
         }
         // park a reached leaf while the slot is free and walk on
         if (s.cur < 0 && s.cur != kNoRef && s.leaf == kNoRef) {
             s.leaf = s.cur;
-            if (s.sp > 0) {
-                --s.sp;
-                s.cur = stack_get(stack, s.sp);
-            } else {
-                s.cur = kNoRef;
-            }
+            --s.sp;
+            s.cur = stack_get(stack, s.sp);
         }
     }
     // leaf phase of the wavefront (the lanes stepping here)
     const bool want = s.leaf != kNoRef;
     const bool stuck = want && s.cur < 0;  // a second leaf, or nothing left to walk
-    if (__ballot(stuck) != 0 || (uint32_t)__popcll(__ballot(want)) >= (ANY ? kLeafBatchAny : kLeafBatch)) {
+    if (__ballot(stuck) != 0 || (uint32_t)__popcll(__ballot(want)) >= leaf_batch) {
         if (want) {
             uint32_t first, count;
             decode_leaf(s.leaf, first, count);
@@ -496,9 +539,10 @@ __device__ __forceinline__ bool trav_step4(TravState &s, const float4 *__restric
 template <bool WIDE, bool ANY, bool STATS, class Stack, bool OPAQUE = false>
 __device__ __forceinline__ bool trav_step_any(TravState &s, const float4 *__restrict__ nodes,
                                               const float4 *__restrict__ tris, const Stack &stack, int cap,
-                                              uint32_t &n_node, uint32_t &n_tri)
+                                              uint32_t leaf_batch, uint32_t &n_node, uint32_t &n_tri)
 {
-    if constexpr (WIDE) return trav_step4<ANY, STATS, Stack, OPAQUE>(s, nodes, tris, stack, cap, n_node, n_tri);
+    if constexpr (WIDE)
+        return trav_step4<ANY, STATS, Stack, OPAQUE>(s, nodes, tris, stack, cap, leaf_batch, n_node, n_tri);
     else return trav_step<ANY, STATS, Stack, OPAQUE>(s, nodes, tris, stack, cap, n_node, n_tri);
 }
 
@@ -534,6 +578,7 @@ struct StripeCursor {
     uint32_t n;       // items in that stripe
     uint32_t salt;    // per-wavefront pseudo-random state for picking a stripe to help
     uint32_t left;    // items of stripe s not yet claimed, as last seen (an upper bound)
+    uint32_t width;   // lanes that take items (64, or fewer when the launch has few items)
     uint32_t wlog;    // log2 of the launch's wavefronts per stripe (rounded down)
     uint32_t ls, lb, le;  // claimed, not yet handed out: items [lb, le) of stripe ls
     bool empty;       // all of stripe s is claimed: scan before the next claim
@@ -544,11 +589,25 @@ struct StripeCursor {
 // is handed out.
 __device__ __forceinline__ bool cursor_finished(const StripeCursor &c) { return c.done && c.lb == c.le; }
 
+// A launch with fewer items than kWidthWaves full wavefronts (two per SIMD)
+// takes them with fewer lanes of more wavefronts, down to kMinWidth: a small
+// launch is as long as its slowest wavefront, and a wavefront runs through the
+// node and leaf work of all its rays in turn.  8192 rays against 4096
+// triangles, closest and any hit: 248 us with 64 lanes, 224 with 16, 214 with
+// 4; cached 960x540 frames 7.28 and 7.03 ms with 64 and 4.
+constexpr uint32_t kWidthWaves = 2048, kMinWidth = 4;
 template <class Count>
 __device__ __forceinline__ void cursor_init(StripeCursor &c, uint32_t home, Count count)
 {
+    const uint32_t mine = count(__lane_id());
+    uint32_t total = mine;
+#pragma unroll
+    for (int off = 32; off > 0; off >>= 1) total += (uint32_t)__shfl_xor((int)total, off);
+    const uint32_t waves = min(gridDim.x * (blockDim.x >> 6), kWidthWaves);
+    c.width = 64u;
+    while (c.width > kMinWidth && total <= (c.width >> 1) * waves) c.width >>= 1;
     c.s = home;
-    c.n = count(home);
+    c.n = (uint32_t)__shfl((int)mine, (int)home);
     c.left = c.n;
     const uint32_t per_stripe = (gridDim.x * (blockDim.x >> 6)) / kStripes;
     c.wlog = per_stripe ? 31u - (uint32_t)__clz(per_stripe) : 0u;
@@ -556,9 +615,12 @@ __device__ __forceinline__ void cursor_init(StripeCursor &c, uint32_t home, Coun
     c.ls = home;
     c.lb = 0;
     c.le = 0;
-    c.empty = false;
-    c.done = false;
+    c.empty = c.n == 0;
+    c.done = total == 0;
 }
+
+// Lanes at a parked leaf that start a leaf phase: a quarter of those that take items.
+__device__ __forceinline__ uint32_t leaf_batch(const StripeCursor &c) { return c.width >> 2; }
 
 // One pass over every stripe's claim counter (lane j reads stripe j): move
 // to a stripe with unclaimed items, drawn at random among them so that the
@@ -600,8 +662,8 @@ __device__ __forceinline__ bool cursor_scan(StripeCursor &c, uint32_t *fetch, Co
 // Items of the next claim (wavefront-uniform).
 __device__ __forceinline__ uint32_t claim_size(const StripeCursor &c)
 {
-    const uint32_t k = c.left >> c.wlog;
-    return k < kClaimMin ? kClaimMin : (k > kClaimChunk ? kClaimChunk : k);
+    const uint32_t k = c.left >> c.wlog, least = min(kClaimMin, c.width);
+    return k < least ? least : (k > kClaimChunk ? kClaimChunk : k);
 }
 
 // Wavefront-uniform refill of idle lanes: when at least kRefillLanes lanes
@@ -615,10 +677,10 @@ template <class Count>
 __device__ __forceinline__ uint32_t wave_claim(StripeCursor &c, uint32_t *fetch, Count count, bool has,
                                                uint32_t &stripe)
 {
-    const uint64_t idle = __ballot(!has);
-    const uint32_t nidle = (uint32_t)__popcll(idle);
-    if (!(nidle >= kRefillLanes || nidle == 64u)) return 0xffffffffu;
     const uint32_t lane = __lane_id();
+    const uint64_t idle = __ballot(!has && lane < c.width);
+    const uint32_t nidle = (uint32_t)__popcll(idle);
+    if (nidle < (c.width * kRefillLanes) >> 6) return 0xffffffffu;
     if (c.lb == c.le) {
         if (c.done) return 0xffffffffu;
         const uint32_t leader = (uint32_t)(__ffsll((unsigned long long)idle) - 1);
@@ -644,7 +706,7 @@ __device__ __forceinline__ uint32_t wave_claim(StripeCursor &c, uint32_t *fetch,
     const uint32_t b0 = c.lb;
     c.lb += take;
     stripe = c.ls;
-    if (has) return 0xffffffffu;
+    if (has || lane >= c.width) return 0xffffffffu;
     const uint32_t r = (uint32_t)__popcll(idle & ((1ull << lane) - 1ull));
     return r < take ? b0 + r : 0xffffffffu;
 }

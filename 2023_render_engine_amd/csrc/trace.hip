@@ -48,6 +48,7 @@ __global__ __launch_bounds__(kTraceBlock) void k_trace(const float4 *__restrict_
     extern __shared__ int32_t s_stack[];
     StackTail<TraceStack> s_tail;
     const TraceStack stack{s_stack + threadIdx.x, s_tail};
+    stack_init(stack);
     // the rays are dealt to the stripes in chunks of 2^lc consecutive rays
     // (chunk c to stripe c % kStripes), so every stripe holds a sample of
     // the whole batch and the stripes take about equally long
@@ -79,7 +80,7 @@ __global__ __launch_bounds__(kTraceBlock) void k_trace(const float4 *__restrict_
             if (cursor_finished(cur)) break;
             continue;
         }
-        if (has && trav_step_any<WIDE, ANY, STATS, TraceStack, OPAQUE>(s, nodes, tris, stack, cap, n_node, n_tri)) {
+        if (has && trav_step_any<WIDE, ANY, STATS, TraceStack, OPAQUE>(s, nodes, tris, stack, cap, leaf_batch(cur), n_node, n_tri)) {
             if (ANY) {
                 occluded[ray] = s.occ ? 1 : 0;
             } else {
@@ -119,7 +120,7 @@ hipError_t launch_trace(const DevBvh &bvh, const RaysDev &rays, uint32_t n, int3
     if (per_cu > 16) per_cu = 16;
     if (per_cu < 1) per_cu = 1;
     size_t blocks = (size_t)g_cus * per_cu;
-    const size_t need = (n + kTraceBlock - 1) / kTraceBlock;
+    const size_t need = ((size_t)n + 2 * kMinWidth - 1) / (2 * kMinWidth);
     if (blocks > need) blocks = need;
     const dim3 grid((unsigned)blocks);
     const float4 *nd = (const float4 *)bvh.nodes, *tr = (const float4 *)bvh.tris;

@@ -226,3 +226,37 @@ def test_shadow_query_replays_scene_is_visible_through_the_c_abi(rt, orc, gpu_ct
     ids2, _ = bvh.trace_closest(*rays, host=True)
     assert np.any(transparent[ids2[ids2 >= 0]])
     bvh.close()
+
+
+@pytest.mark.parametrize("scale", [1e-3, 1.0, 1e4])
+@pytest.mark.parametrize("n", [1, 3, 63, 64, 65, 1000, 9001])
+def test_small_launches_and_axis_parallel_rays(rt, orc, gpu_ctx, n, scale):
+    """Launches small enough to use a few lanes of each wavefront, with rays
+    along the axes (zero direction components) mixed in, in scenes of other
+    sizes: ids and distances equal brute force on unambiguous rays, and any
+    hit agrees with the closest one."""
+    xyz, idx = rt.gen_soup(3000, seed=5, edge_mu=0.05)
+    xyz = (xyz * np.float32(scale)).astype(np.float32)
+    rays = [a.copy() for a in rt.gen_rays(1, 1, n_incoherent=n + 8, seed=n)]
+    rays = [a[:n].copy() for a in rays]
+    for k in range(3):
+        rays[k] = (rays[k] * np.float32(scale)).astype(np.float32)
+    for k in range(0, n, 3):  # along an axis, both ways, and in a coordinate plane
+        d = np.zeros(3, np.float32)
+        d[(k // 3) % 3] = 1.0 if k % 2 else -1.0
+        if k % 4 == 0:
+            d[(k // 3 + 1) % 3] = 0.5
+        for c in range(3):
+            rays[3 + c][k] = d[c]
+    bvh = rt.Bvh(gpu_ctx, xyz, idx)
+    prim, t = bvh.trace_closest(*to_dev(rays))
+    bp, bt, fl = orc.brute_trace(xyz, idx, rays)
+    clean = fl == 0
+    torch.cuda.synchronize()
+    prim, t = prim.cpu().numpy(), t.cpu().numpy()
+    assert np.array_equal(prim[clean], bp[clean])
+    assert np.array_equal(t[clean], bt[clean])
+    tmax = np.where(bp >= 0, bt * np.float32(1.5), np.float32(10 * scale)).astype(np.float32)
+    occ = bvh.trace_any(*to_dev(rays), torch.from_numpy(tmax).cuda())
+    torch.cuda.synchronize()
+    assert np.array_equal(occ.cpu().numpy()[clean].astype(bool), bp[clean] >= 0)
