@@ -5,13 +5,16 @@
 //   extend   closest hit (BVH + analytic spheres) for every active path,
 //            then material classification into per-class queues with
 //            wavefront ballots (one atomic per 64 lanes per queue);
-//   shade<M> one kernel per material class (Lambertian, dielectric, GGX,
+//   shade    one workgroup per material class (Lambertian, dielectric, GGX,
 //            light, miss), so a wavefront runs a single BSDF: resolves the
 //            previous bounce's next-event estimate, emits this bounce's
 //            shadow rays, samples the BSDF, applies Russian roulette and
 //            appends survivors to the next active queue;
 //   connect  any hit for every shadow ray; occluded rays clear their light
 //            bit in the path's NEE mask;
+//   regen    the paths that ended give their radiance and their slots take the
+//            chunk's next paths;
+//   commit   one wavefront: counts, statistics and resets for the next bounce;
 // and a final pass adds finished paths to the FP64 film.
 //
 // The estimator is the reference's (integration/pathTracing.cu:33-123,
@@ -41,7 +44,6 @@ namespace rt {
 
 constexpr int kBlock = 128;
 constexpr int kGrid = 2048;  // 8 workgroups per CU on 256 CUs
-
 __device__ __forceinline__ uint32_t wave_append(uint32_t *counter, bool pred)
 {
     const uint64_t mask = __ballot(pred);
@@ -156,21 +158,14 @@ __device__ __forceinline__ Pcg32 path_rng(float4 q, uint64_t stream_base)
 }
 
 // ---------------------------------------------------------------------
-// Counter resets.  Per iteration: the next live list, the material queues,
-// the shadow list, the terminated list, the claim counters of the
-// persistent kernels and the cache queries; at a chunk's start: all.
-// Workgroup L < kNumLists clears list L's stripe counters (one lane per
-// stripe), the last workgroup the scalar counters.
-__global__ __launch_bounds__(kStripes) void k_reset(QueuesDev q, uint32_t cur, uint32_t chunk_start)
+// Counter reset at a chunk's start: workgroup L < kNumLists clears list L's
+// stripe counters (one lane per stripe), the last workgroup the scalar
+// counters.  (Between iterations k_commit clears what the next one fills.)
+__global__ __launch_bounds__(kStripes) void k_reset(QueuesDev q)
 {
     const uint32_t L = blockIdx.x, t = threadIdx.x;
-    if (L < kNumLists) {
-        const bool clear = chunk_start || L == kLActive0 + (cur ^ 1u) || (L >= kLQueue && L <= kLTerm) ||
-                           L == kLClaimExt || L == kLClaimCon;
-        if (clear) *lcount(q, L, t) = 0;
-    } else if (t < kNumCounters && (chunk_start || t == kCCacheQ)) {
-        *scount(q, t) = 0;
-    }
+    if (L < kNumLists) *lcount(q, L, t) = 0;
+    else if (t < kNumCounters) *scount(q, t) = 0;
 }
 
 // A new path in `slot`: global path index g (chunk index k).  Within its
@@ -236,7 +231,7 @@ __device__ __forceinline__ void init_path(const SceneDev &sc0, const BatchDev &b
 // stripe's next live list after its surviving paths.  At a chunk's start
 // stripe s takes chunk paths s, s + 64, s + 128, ... (balanced stripes);
 // later, the stripes' free slots in stripe order take the chunk's next
-// paths in order.  No atomics: k_regen_commit advances the counters after.
+// paths in order.  No atomics: k_commit advances the counters after.
 // Called by whole wavefronts (lane j reads stripe j's free count).
 struct RegenPlan {
     uint32_t next;   // chunk paths handed out before this regeneration
@@ -268,38 +263,129 @@ __device__ __forceinline__ RegenPlan regen_plan(const QueuesDev &q, const WavePa
     return r;
 }
 
-template <bool B>
+// The radiance L after adding the previous bounce's unoccluded next-event
+// contributions (mask: their light slots), in light order, times the
+// throughput nb they were computed with.
+__device__ __forceinline__ V3 resolved_L(const PathsDev &p, uint32_t slot, uint32_t mask, V3 L, V3 nb)
+{
+    if (mask == 0) return L;
+    V3 Ld = mk(0, 0, 0);
+    const float *c = p.nee_c + (size_t)slot * p.nee_stride * 3;
+    while (mask) {
+        const uint32_t l = __ffs(mask) - 1;
+        mask &= mask - 1;
+        Ld = add(Ld, mk(c[3 * l], c[3 * l + 1], c[3 * l + 2]));
+    }
+    return mk(L.x + nb.x * Ld.x, L.y + nb.y * Ld.y, L.z + nb.z * Ld.z);
+}
+
+// What k_regen does with the paths that ended: their results, and the
+// training records of training (wp.train) and harvesting waves (up to cap).
+struct FinalizeArgs {
+    float *res;
+    uint32_t harvest, cap;
+};
+
+// A path that ended this iteration takes its last next-event contributions.
+// Rendering: the radiance goes to res[path index].  Training: a path that
+// passed a cacheable vertex at the cache depth yields the target
+// (L_end - L_arrival) / beta_arrival per channel (0 where beta is 0),
+// compacted with its record into cin / ttgt; non-finite targets are dropped.
+// Called by whole wavefronts.
+__device__ __forceinline__ void finalize_path(const PathsDev &p, const QueuesDev &q, const FinalizeArgs &f,
+                                              uint32_t train, uint32_t slot, bool live)
+{
+    V3 L = mk(0, 0, 0);
+    uint32_t tvalid = 0;
+    float4 qL{};
+    if (live) {
+        const float4 *rec = path_rec(p, slot);
+        qL = rec[kPqL];
+        const float4 qn = rec[kPqNee];
+        L = resolved_L(p, slot, bits(rec[kPqRng].w), mk(qL.x, qL.y, qL.z), mk(qn.x, qn.y, qn.z));
+        tvalid = bits(qn.w);
+    }
+    if (!train && live) {
+        float *r = f.res + 3 * (size_t)bits(qL.w);
+        r[0] = L.x; r[1] = L.y; r[2] = L.z;
+    }
+    if (!train && !f.harvest) return;  // wavefront-uniform (kernel arguments)
+    bool ok = false;
+    float tg[3] = {0, 0, 0};
+    if (live && tvalid) {
+        const float Le[3] = {L.x, L.y, L.z};
+        ok = true;
+        for (int c = 0; c < 3; ++c) {
+            const float b = p.tB[3 * (size_t)slot + c];
+            tg[c] = b > 0 ? (Le[c] - p.tLb[3 * (size_t)slot + c]) / b : 0.0f;
+            ok = ok && isfinite(tg[c]);
+        }
+    }
+    const uint32_t k = wave_append(scount(q, kCTrain), ok);
+    if (ok && k < f.cap) {
+        const float4 *src = (const float4 *)(p.tin + (size_t)slot * 12);
+        float4 *dst = (float4 *)(p.cin + (size_t)k * 12);
+        dst[0] = src[0]; dst[1] = src[1]; dst[2] = src[2];
+        p.ttgt[3 * (size_t)k] = fmaxf(tg[0], 0.0f);
+        p.ttgt[3 * (size_t)k + 1] = fmaxf(tg[1], 0.0f);
+        p.ttgt[3 * (size_t)k + 2] = fmaxf(tg[2], 0.0f);
+    }
+}
+
+// INIT: a chunk's start.  Otherwise the lane that ends a path also starts the
+// next one in its slot, so the two need no launch or list of their own.
+template <bool B, bool INIT>
 __global__ __launch_bounds__(kBlock) void k_regen(SceneDev sc0, BatchDev bt, PathsDev p, QueuesDev q, WaveParams wp,
-                                                  uint32_t nxt, uint32_t init, uint32_t capacity)
+                                                  uint32_t nxt, uint32_t capacity, FinalizeArgs fin)
 {
     const uint64_t first = wp.chunk_dev ? wp.chunk_dev[0] : wp.first_path;
     const StripeSpan sp = stripe_span();
     const uint32_t s = sp.s, cs = q.cs;
-    const RegenPlan r = regen_plan(q, wp, init, capacity, s);
+    const RegenPlan r = regen_plan(q, wp, INIT ? 1u : 0u, capacity, s);
     const uint32_t n_live = *lcount(q, kLActive0 + nxt, s);
-    for (uint32_t j = sp.j0 + threadIdx.x; j < r.take; j += sp.step) {
-        const uint32_t slot = init ? s * cs + j : q.term[s * cs + j];
-        const uint32_t k = r.next + (init ? j * kStripes + s : r.pre + j);
-        init_path<B>(sc0, bt, p, wp, slot, first + k, k);
-        q.active[nxt][s * cs + n_live + j] = slot;
+    const uint32_t n = INIT ? r.take : *lcount(q, kLTerm, s);
+    for (uint32_t j0 = sp.j0; j0 < n; j0 += sp.step) {
+        const uint32_t j = j0 + threadIdx.x;
+        const bool live = j < n;
+        const uint32_t slot = INIT ? s * cs + j : (live ? q.term[s * cs + j] : 0u);
+        if (!INIT) finalize_path(p, q, fin, wp.train, slot, live);
+        if (j < r.take) {
+            const uint32_t k = r.next + (INIT ? j * kStripes + s : r.pre + j);
+            init_path<B>(sc0, bt, p, wp, slot, first + k, k);
+            q.active[nxt][s * cs + n_live + j] = slot;
+        }
     }
 }
 
 // One wavefront, lane s = stripe s: the stripes' live counts grow by what
 // they took; the next unclaimed path and the total live count (for the
-// host's end-of-chunk test) are updated.
-__global__ __launch_bounds__(kStripes) void k_regen_commit(QueuesDev q, WaveParams wp, uint32_t nxt, uint32_t init,
-                                                           uint32_t capacity)
+// host's end-of-chunk test) are updated.  After an iteration (init = 0) it
+// also adds the iteration's rays to the statistics and clears what the next
+// iteration fills: the live list it walked, the material queues, the shadow
+// and terminated lists, the claim counters and the cache queries.
+__global__ __launch_bounds__(kStripes) void k_commit(QueuesDev q, WaveParams wp, uint32_t nxt, uint32_t init,
+                                                     uint32_t capacity)
 {
     const uint32_t s = threadIdx.x;
     const RegenPlan r = regen_plan(q, wp, init, capacity, s);
-    uint32_t *live = lcount(q, kLActive0 + nxt, s);
+    uint32_t *live = lcount(q, kLActive0 + nxt, s), *old = lcount(q, kLActive0 + (nxt ^ 1u), s);
     const uint32_t n = *live + r.take;
     const uint32_t total = wave_sum(n);
+    const uint32_t ext = wave_sum(*old), shd = wave_sum(*lcount(q, kLShadow, s));
     *live = n;
     if (s == 0) {
         *scount(q, kCNext) = r.next + r.n_new;
         *scount(q, kCLive) = total;
+        if (!init) {
+            q.stats[kStatExt] += ext;
+            q.stats[kStatShadow] += shd;
+            *scount(q, kCCacheQ) = 0;
+        }
+    }
+    if (!init) {
+        *old = 0;
+#pragma unroll
+        for (uint32_t L = kLQueue; L < kNumLists; ++L) *lcount(q, L, s) = 0;
     }
 }
 
@@ -481,22 +567,6 @@ __global__ __launch_bounds__(kBlock) void k_classify(SceneDev sc0, BatchDev bt, 
 // ---------------------------------------------------------------------
 // shading
 // ---------------------------------------------------------------------
-// The radiance L after adding the previous bounce's unoccluded next-event
-// contributions (mask: their light slots), in light order, times the
-// throughput nb they were computed with.
-__device__ __forceinline__ V3 resolved_L(const PathsDev &p, uint32_t slot, uint32_t mask, V3 L, V3 nb)
-{
-    if (mask == 0) return L;
-    V3 Ld = mk(0, 0, 0);
-    const float *c = p.nee_c + (size_t)slot * p.nee_stride * 3;
-    while (mask) {
-        const uint32_t l = __ffs(mask) - 1;
-        mask &= mask - 1;
-        Ld = add(Ld, mk(c[3 * l], c[3 * l + 1], c[3 * l + 2]));
-    }
-    return mk(L.x + nb.x * Ld.x, L.y + nb.y * Ld.y, L.z + nb.z * Ld.z);
-}
-
 // resolved_L in place: the record's radiance takes the contributions and its
 // mask is cleared.
 __device__ __forceinline__ void resolve_nee(const PathsDev &p, uint32_t slot)
@@ -543,11 +613,11 @@ __device__ __forceinline__ void write_record(float *r, const Surface &s, V3 d, c
 }
 
 template <uint32_t CLS, bool B>
-__global__ __launch_bounds__(kBlock) void k_shade(SceneDev sc0, BatchDev bt, PathsDev p, ShadowDev sh, QueuesDev q,
-                                                  WaveParams wp, uint32_t cur)
+__device__ __forceinline__ void shade_class(const SceneDev &sc0, const BatchDev &bt, const PathsDev &p,
+                                            const ShadowDev &sh, const QueuesDev &q, const WaveParams &wp,
+                                            uint32_t cur, const StripeSpan &sp)
 {
     constexpr bool kScatter = CLS == kQLambert || CLS == kQGgx;
-    const StripeSpan sp = stripe_span();
     const uint32_t cs = q.cs, base = sp.s * cs;
     const uint32_t n = *lcount(q, kLQueue + CLS, sp.s);
     const uint32_t *queue = q.q[CLS] + base;
@@ -766,6 +836,26 @@ __global__ __launch_bounds__(kBlock) void k_shade(SceneDev sc0, BatchDev bt, Pat
     }
 }
 
+// All five classes in one launch: workgroup b serves stripe b % kStripes and
+// class b / kStripes % 5, so a wavefront still runs one material.  The
+// classes overlap, which is worth more than each one's own register count
+// (154 for GGX): against five launches the preview frame (333x187, 1 spp)
+// takes 1.40 instead of 1.69 ms, the Cornell box (256x256, 16 spp) 1.68
+// instead of 1.85, a 1080p frame of 64 spp 254.6 instead of 266.6.
+template <bool B>
+__global__ __launch_bounds__(kBlock) void k_shade(SceneDev sc0, BatchDev bt, PathsDev p, ShadowDev sh, QueuesDev q,
+                                                  WaveParams wp, uint32_t cur)
+{
+    const uint32_t c = blockIdx.x / kStripes % 5u;
+    const StripeSpan sp{blockIdx.x % kStripes, blockIdx.x / (5u * kStripes) * kBlock,
+                        gridDim.x / (5u * kStripes) * kBlock};
+    if (c == 0) shade_class<kQLambert, B>(sc0, bt, p, sh, q, wp, cur, sp);
+    else if (c == 1) shade_class<kQGgx, B>(sc0, bt, p, sh, q, wp, cur, sp);
+    else if (c == 2) shade_class<kQDielectric, B>(sc0, bt, p, sh, q, wp, cur, sp);
+    else if (c == 3) shade_class<kQLight, B>(sc0, bt, p, sh, q, wp, cur, sp);
+    else shade_class<kQMiss, B>(sc0, bt, p, sh, q, wp, cur, sp);
+}
+
 // Cache vertices: the path ends here.  Its previous next-event estimate is
 // resolved and its query record is written to the iteration's query rows;
 // the cache's answer times the throughput on arrival is added after the
@@ -931,63 +1021,6 @@ __global__ __launch_bounds__(kBlock) void k_connect(SceneDev sc0, BatchDev bt, P
     }
 }
 
-// ---------------------------------------------------------------------
-// finalize: paths that ended this iteration take their last next-event
-// contributions.  Rendering: the radiance goes to res[path index].
-// Training: a path that passed a cacheable vertex at the cache depth yields
-// the target (L_end - L_arrival) / beta_arrival per channel (0 where beta is
-// 0), compacted with its record into cin / ttgt; non-finite targets are
-// dropped.
-// ---------------------------------------------------------------------
-__global__ __launch_bounds__(kBlock) void k_finalize(PathsDev p, QueuesDev q, float *res, uint32_t train,
-                                                    uint32_t harvest, uint32_t cap)
-{
-    const StripeSpan sp = stripe_span();
-    const uint32_t n = *lcount(q, kLTerm, sp.s);
-    const uint32_t *term = q.term + sp.s * q.cs;
-    for (uint32_t j0 = sp.j0; j0 < n; j0 += sp.step) {
-        const uint32_t i = j0 + threadIdx.x;
-        const bool live = i < n;
-        const uint32_t slot = live ? term[i] : 0;
-        // the slot is refilled next, so the resolved radiance stays in registers
-        V3 L = mk(0, 0, 0);
-        uint32_t tvalid = 0;
-        float4 qL{};
-        if (live) {
-            const float4 *rec = path_rec(p, slot);
-            qL = rec[kPqL];
-            const float4 qn = rec[kPqNee];
-            L = resolved_L(p, slot, bits(rec[kPqRng].w), mk(qL.x, qL.y, qL.z), mk(qn.x, qn.y, qn.z));
-            tvalid = bits(qn.w);
-        }
-        if (!train && live) {
-            float *r = res + 3 * (size_t)bits(qL.w);
-            r[0] = L.x; r[1] = L.y; r[2] = L.z;
-        }
-        if (!train && !harvest) continue;  // wavefront-uniform (kernel arguments)
-        bool ok = false;
-        float tg[3] = {0, 0, 0};
-        if (live && tvalid) {
-            const float Le[3] = {L.x, L.y, L.z};
-            ok = true;
-            for (int c = 0; c < 3; ++c) {
-                const float b = p.tB[3 * (size_t)slot + c];
-                tg[c] = b > 0 ? (Le[c] - p.tLb[3 * (size_t)slot + c]) / b : 0.0f;
-                ok = ok && isfinite(tg[c]);
-            }
-        }
-        const uint32_t k = wave_append(scount(q, kCTrain), ok);
-        if (ok && k < cap) {
-            const float4 *src = (const float4 *)(p.tin + (size_t)slot * 12);
-            float4 *dst = (float4 *)(p.cin + (size_t)k * 12);
-            dst[0] = src[0]; dst[1] = src[1]; dst[2] = src[2];
-            p.ttgt[3 * (size_t)k] = fmaxf(tg[0], 0.0f);
-            p.ttgt[3 * (size_t)k + 1] = fmaxf(tg[1], 0.0f);
-            p.ttgt[3 * (size_t)k + 2] = fmaxf(tg[2], 0.0f);
-        }
-    }
-}
-
 // L += beta * cache(record) for this iteration's cache queries; the paths
 // ended at their cache vertex and are finalized right after
 __global__ __launch_bounds__(kBlock) void k_cache_apply(PathsDev p, QueuesDev q)
@@ -1031,18 +1064,6 @@ __global__ __launch_bounds__(kBlock) void k_film(const float *res, FilmDev film,
         film.accum[3 * (size_t)px + 1] += sy;
         film.accum[3 * (size_t)px + 2] += sz;
         film.nvalid[px] += nv;
-    }
-}
-
-// Ray statistics of an iteration (one wavefront, lane s = stripe s).
-__global__ __launch_bounds__(kStripes) void k_count(QueuesDev q, uint32_t cur)
-{
-    const uint32_t s = threadIdx.x;
-    const uint32_t ext = wave_sum(*lcount(q, kLActive0 + cur, s));
-    const uint32_t shd = wave_sum(*lcount(q, kLShadow, s));
-    if (s == 0) {
-        q.stats[0] += ext;
-        q.stats[1] += shd;
     }
 }
 
@@ -1116,10 +1137,11 @@ hipError_t chunk_begin(const ChunkLaunch &c, const WaveParams &wp, hipStream_t s
     const dim3 grid = queue_grid(wp);
     const SceneDev &sc = *c.scene;
     const BatchDev bt = c.batch ? c.batch->dev : BatchDev{nullptr, nullptr, 0, nullptr, nullptr, nullptr, nullptr};
-    hipLaunchKernelGGL(k_reset, dim3(kNumLists + 1), dim3(kStripes), 0, s, q, 0u, 1u);
-    if (c.batch) hipLaunchKernelGGL(k_regen<true>, grid, blk, 0, s, sc, bt, c.paths, q, wp, 0u, 1u, c.capacity);
-    else hipLaunchKernelGGL(k_regen<false>, grid, blk, 0, s, sc, bt, c.paths, q, wp, 0u, 1u, c.capacity);
-    hipLaunchKernelGGL(k_regen_commit, dim3(1), dim3(kStripes), 0, s, q, wp, 0u, 1u, c.capacity);
+    const FinalizeArgs none{nullptr, 0, 0};
+    hipLaunchKernelGGL(k_reset, dim3(kNumLists + 1), dim3(kStripes), 0, s, q);
+    if (c.batch) hipLaunchKernelGGL((k_regen<true, true>), grid, blk, 0, s, sc, bt, c.paths, q, wp, 0u, c.capacity, none);
+    else hipLaunchKernelGGL((k_regen<false, true>), grid, blk, 0, s, sc, bt, c.paths, q, wp, 0u, c.capacity, none);
+    hipLaunchKernelGGL(k_commit, dim3(1), dim3(kStripes), 0, s, q, wp, 0u, 1u, c.capacity);
     return hipGetLastError();
 }
 
@@ -1179,37 +1201,32 @@ hipError_t chunk_iterate(const ChunkLaunch &c, const WaveParams &wp, uint32_t it
         else if (wide) cnt ? go(k_connect<false, true, true>) : go(k_connect<false, true, false>);
         else cnt ? go(k_connect<false, false, true>) : go(k_connect<false, false, false>);
     };
+    // workgroups per class and stripe: enough for every item of a small wave, at
+    // most 256 (1080p frame at 16, 32, 64, 256 and 2048: 262.6, 257.2, 254.3,
+    // 251.1, 254.5 ms), scaled with the grid option
+    const uint32_t most = std::max(1u, (wp.grid ? wp.grid : (uint32_t)kGrid) / 8u);
+    const dim3 sgrid(5u * kStripes * std::min((q.cs + kBlock - 1) / kBlock, most));
     for (uint32_t it = 0; it < iterations; ++it) {
         const uint32_t nxt = cur ^ 1u;
-        hipLaunchKernelGGL(k_reset, dim3(kNumLists + 1), dim3(kStripes), 0, s, q, cur, 0u);
         timed(0, extend);
         if (B) {
             hipLaunchKernelGGL(k_classify<true>, grid, blk, 0, s, sc, bt, paths, q, cur, ext_depth, need_record, 0u);
-            hipLaunchKernelGGL((k_shade<kQLambert, true>), grid, blk, 0, s, sc, bt, paths, shadow, q, wp, cur);
-            hipLaunchKernelGGL((k_shade<kQDielectric, true>), grid, blk, 0, s, sc, bt, paths, shadow, q, wp, cur);
-            hipLaunchKernelGGL((k_shade<kQGgx, true>), grid, blk, 0, s, sc, bt, paths, shadow, q, wp, cur);
-            hipLaunchKernelGGL((k_shade<kQLight, true>), grid, blk, 0, s, sc, bt, paths, shadow, q, wp, cur);
-            hipLaunchKernelGGL((k_shade<kQMiss, true>), grid, blk, 0, s, sc, bt, paths, shadow, q, wp, cur);
+            hipLaunchKernelGGL((k_shade<true>), sgrid, blk, 0, s, sc, bt, paths, shadow, q, wp, cur);
         } else {
             hipLaunchKernelGGL(k_classify<false>, grid, blk, 0, s, sc, bt, paths, q, cur, ext_depth, need_record,
                                photon ? (c.photon->hybrid ? 2u : 1u) : 0u);
             // hybrid queries record the throughput on arrival, before shading
             if (photon && c.photon->hybrid)
                 hipLaunchKernelGGL(k_photon_vertex<true>, grid, blk, 0, s, sc, paths, q, *c.photon);
-            hipLaunchKernelGGL((k_shade<kQLambert, false>), grid, blk, 0, s, sc, bt, paths, shadow, q, wp, cur);
-            hipLaunchKernelGGL((k_shade<kQDielectric, false>), grid, blk, 0, s, sc, bt, paths, shadow, q, wp, cur);
-            hipLaunchKernelGGL((k_shade<kQGgx, false>), grid, blk, 0, s, sc, bt, paths, shadow, q, wp, cur);
-            hipLaunchKernelGGL((k_shade<kQLight, false>), grid, blk, 0, s, sc, bt, paths, shadow, q, wp, cur);
-            hipLaunchKernelGGL((k_shade<kQMiss, false>), grid, blk, 0, s, sc, bt, paths, shadow, q, wp, cur);
+            hipLaunchKernelGGL((k_shade<false>), sgrid, blk, 0, s, sc, bt, paths, shadow, q, wp, cur);
         }
         if (lookups) hipLaunchKernelGGL(k_cache_vertex, grid, blk, 0, s, sc, paths, q);
         if (photon && !c.photon->hybrid)
             hipLaunchKernelGGL(k_photon_vertex<false>, grid, blk, 0, s, sc, paths, q, *c.photon);
-        hipLaunchKernelGGL(k_count, dim3(1), dim3(kStripes), 0, s, q, cur);
         timed(1, connect);
         if (lookups) {
             // cin rows are this iteration's queries (training records are
-            // compacted into cin only by k_finalize, after this)
+            // compacted into cin only by k_regen, after this)
             hipError_t e = cache_infer(*c.cache, paths.cqin, c.capacity, paths.crgb, s,
                                        scount(q, kCCacheQ));
             if (e != hipSuccess) return e;
@@ -1224,11 +1241,10 @@ hipError_t chunk_iterate(const ChunkLaunch &c, const WaveParams &wp, uint32_t it
             else hipLaunchKernelGGL(k_photon_apply<false>, grid, blk, 0, s, paths, q, ph);
         }
         const uint32_t harvest = wp.harvest_shift != kNoHarvest ? 1u : 0u;
-        const uint32_t cap = wp.train ? c.capacity : (harvest ? wp.harvest_cap : 0u);
-        hipLaunchKernelGGL(k_finalize, grid, blk, 0, s, paths, q, c.res, wp.train, harvest, cap);
-        if (B) hipLaunchKernelGGL(k_regen<true>, grid, blk, 0, s, sc, bt, paths, q, wp, nxt, 0u, c.capacity);
-        else hipLaunchKernelGGL(k_regen<false>, grid, blk, 0, s, sc, bt, paths, q, wp, nxt, 0u, c.capacity);
-        hipLaunchKernelGGL(k_regen_commit, dim3(1), dim3(kStripes), 0, s, q, wp, nxt, 0u, c.capacity);
+        const FinalizeArgs fin{c.res, harvest, wp.train ? c.capacity : (harvest ? wp.harvest_cap : 0u)};
+        if (B) hipLaunchKernelGGL((k_regen<true, false>), grid, blk, 0, s, sc, bt, paths, q, wp, nxt, c.capacity, fin);
+        else hipLaunchKernelGGL((k_regen<false, false>), grid, blk, 0, s, sc, bt, paths, q, wp, nxt, c.capacity, fin);
+        hipLaunchKernelGGL(k_commit, dim3(1), dim3(kStripes), 0, s, q, wp, nxt, 0u, c.capacity);
         cur = nxt;
     }
     return hipGetLastError();

@@ -616,7 +616,9 @@ __device__ __forceinline__ void cursor_init(StripeCursor &c, uint32_t home, Coun
     c.lb = 0;
     c.le = 0;
     c.empty = c.n == 0;
-    c.done = total == 0;
+    // in a small launch a stripe's own wavefronts suffice: the rest leave
+    const uint32_t nth = (blockIdx.x / kStripes) * (blockDim.x >> 6) + (threadIdx.x >> 6);
+    c.done = total == 0 || (c.width < 64u && nth * c.width >= c.n);
 }
 
 // Lanes at a parked leaf that start a leaf phase: a quarter of those that take items.

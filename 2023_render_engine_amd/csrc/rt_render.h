@@ -170,7 +170,7 @@ struct WaveParams {
     // harvesting (rendering waves): one path in 2^harvest_shift (by a hash of
     // its global index; kNoHarvest: none) ignores the cache, and its first
     // cacheable vertex at cache_depth or deeper becomes a training record;
-    // k_finalize compacts up to harvest_cap records into cin / ttgt
+    // k_regen compacts up to harvest_cap records into cin / ttgt
     uint32_t harvest_shift = 0xffffffffu;  // kNoHarvest
     uint32_t harvest_cap = 0;
     float nee_scale = 1.0f;     // factor of every next-event term (RENDER_MODE HYBRID: 0.5)
