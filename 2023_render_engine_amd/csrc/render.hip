@@ -612,6 +612,18 @@ __device__ __forceinline__ void write_record(float *r, const Surface &s, V3 d, c
     r[10] = 0; r[11] = 0;
 }
 
+// Origin of the shadow rays of a vertex.  Every light that is sampled lies on
+// the normal's side, so spawnRay's origin is the same for all of them.
+__device__ __forceinline__ V3 light_origin(const Surface &s) { return spawn_origin(s.p, s.perr, s.n, s.n); }
+
+// Direction and distance of a point light, as shading and its shadow ray use them.
+__device__ __forceinline__ V3 point_light_dir(const rt_point_light &pl, V3 p, V3 &tol, float &dist)
+{
+    tol = sub(mk(pl.pos[0], pl.pos[1], pl.pos[2]), p);
+    dist = len(tol);
+    return nrm(tol);
+}
+
 template <uint32_t CLS, bool B>
 __device__ __forceinline__ void shade_class(const SceneDev &sc0, const BatchDev &bt, const PathsDev &p,
                                             const ShadowDev &sh, const QueuesDev &q, const WaveParams &wp,
@@ -677,21 +689,22 @@ __device__ __forceinline__ void shade_class(const SceneDev &sc0, const BatchDev 
             }
             if (kScatter) {
                 // next-event estimation over every point light (Scene.cu:468-525)
-                // the shadow rays' tree root (batches)
-                const int32_t proot = B && live ? (int32_t)*path_word(p, slot, kPqScene, 1) : 0;
+                // the vertex's place in the stripe: Lambertian ones from the front, GGX
+                // ones from the back (a path is in one class)
+                const uint32_t vert = CLS == kQLambert ? i : cs - 1u - i;
+                const uint32_t psid = B && live ? *path_word(p, slot, kPqScene, 0) : 0u;
                 float *c = p.nee_c + (size_t)slot * p.nee_stride * 3;
                 const uint32_t npl = live ? sc.npl : 0u, nal = live ? sc.nlights - sc.npl : 0u;
                 const uint32_t npl_w = UNI ? sc.npl : wave_max(npl);
                 const uint32_t nal_w = UNI ? sc.nlights - sc.npl : wave_max(nal);
                 for (uint32_t l = 0; l < npl_w; ++l) {
                     bool e = false;
-                    V3 Lw = mk(0, 0, 1), o2 = mk(0, 0, 0);
+                    V3 Lw = mk(0, 0, 1);
                     float dist = 0;
                     if (live && l < npl) {
                         const rt_point_light &pl = uniform_ref<UNI>(sc.pl + l);
-                        const V3 lp = mk(pl.pos[0], pl.pos[1], pl.pos[2]);
-                        const V3 tol = sub(lp, s.p);
-                        Lw = nrm(tol);
+                        V3 tol;
+                        Lw = point_light_dir(pl, s.p, tol, dist);
                         const float d2 = dot(tol, tol);
                         const float I = pl.intensity;
                         const V3 Li = mk(pl.color[0] * I * (1 / d2), pl.color[1] * I * (1 / d2), pl.color[2] * I * (1 / d2));
@@ -704,26 +717,16 @@ __device__ __forceinline__ void shade_class(const SceneDev &sc0, const BatchDev 
                                 c[3 * l] = f.x * Li.x * w * wp.nee_scale;
                                 c[3 * l + 1] = f.y * Li.y * w * wp.nee_scale;
                                 c[3 * l + 2] = f.z * Li.z * w * wp.nee_scale;
-                                dist = len(tol);
-                                o2 = spawn_origin(s.p, s.perr, s.n, Lw);
-                                e = !spheres_occlude(sc, o2, Lw, dist, -1);
+                                e = !spheres_occlude(sc, light_origin(s), Lw, dist, -1);
                             }
                         }
                     }
-                    const size_t pos = sbase + wave_append(lcount(q, kLShadow, sp.s), e);
-                    if (e) {
-                        emit |= 1u << l;
-                        sh.ox[pos] = o2.x; sh.oy[pos] = o2.y; sh.oz[pos] = o2.z;
-                        sh.dx[pos] = Lw.x; sh.dy[pos] = Lw.y; sh.dz[pos] = Lw.z;
-                        sh.tmax[pos] = dist;
-                        sh.slot[pos] = (slot << 5) | l;
-                        if constexpr (B) sh.root[pos] = proot;
-                    }
+                    if (e) emit |= 1u << l;
                 }
                 for (uint32_t a = 0; a < nal_w; ++a) {
                     uint32_t j = 0, l = 0;
                     bool e = false;
-                    V3 Lw = mk(0, 0, 1), o2 = mk(0, 0, 0);
+                    V3 Lw = mk(0, 0, 1);
                     float dist = 0;
                     if (live && a < nal) {
                         j = sc.area_light[a];
@@ -741,19 +744,34 @@ __device__ __forceinline__ void shade_class(const SceneDev &sc0, const BatchDev 
                                 c[3 * l] = f.x * lm.kd[0] * lm.intensity * k * wp.nee_scale;
                                 c[3 * l + 1] = f.y * lm.kd[1] * lm.intensity * k * wp.nee_scale;
                                 c[3 * l + 2] = f.z * lm.kd[2] * lm.intensity * k * wp.nee_scale;
-                                o2 = spawn_origin(s.p, s.perr, s.n, Lw);
-                                e = !spheres_occlude(sc, o2, Lw, dist * 0.9999f, (int32_t)j);
+                                e = !spheres_occlude(sc, light_origin(s), Lw, dist * 0.9999f, (int32_t)j);
                             }
                         }
                     }
-                    const size_t pos = sbase + wave_append(lcount(q, kLShadow, sp.s), e);
                     if (e) {
                         emit |= 1u << l;
-                        sh.ox[pos] = o2.x; sh.oy[pos] = o2.y; sh.oz[pos] = o2.z;
-                        sh.dx[pos] = Lw.x; sh.dy[pos] = Lw.y; sh.dz[pos] = Lw.z;
-                        sh.tmax[pos] = dist * 0.9999f;
-                        sh.slot[pos] = (slot << 5) | l;
-                        if constexpr (B) sh.root[pos] = proot;
+                        sh.area[(size_t)a * cs * kStripes + base + vert] = make_float4(Lw.x, Lw.y, Lw.z, dist * 0.9999f);
+                    }
+                }
+                // the shadow rays: a word each, and the origin and the vertex once
+                // (ShadowDev); one append for the wavefront's rays, light by light
+                if (emit) {
+                    const V3 o2 = light_origin(s);
+                    sh.org[2 * (size_t)(base + vert)] = make_float4(o2.x, o2.y, o2.z, s.p.x);
+                    sh.org[2 * (size_t)(base + vert) + 1] = make_float4(s.p.y, s.p.z, as_f(slot), as_f(psid));
+                }
+                const uint32_t nl_w = npl_w + nal_w;
+                const uint32_t count = wave_sum((uint32_t)__popc(emit));
+                if (count != 0) {
+                    uint32_t at = 0;
+                    if (__lane_id() == 0) at = atomicAdd(lcount(q, kLShadow, sp.s), count);
+                    at = (uint32_t)__builtin_amdgcn_readfirstlane((int)at);
+                    const uint64_t below = (1ull << __lane_id()) - 1ull;
+                    for (uint32_t l = 0; l < nl_w; ++l) {
+                        const bool e = (emit >> l) & 1u;
+                        const uint64_t m = __ballot(e);
+                        if (e) sh.ray[sbase + at + (uint32_t)__popcll(m & below)] = (vert << 5) | l;
+                        at += (uint32_t)__popcll(m);
                     }
                 }
                 // the throughput these estimates were made with
@@ -988,7 +1006,7 @@ __global__ __launch_bounds__(kBlock) void k_connect(SceneDev sc0, BatchDev bt, P
     cursor_init(c, blockIdx.x % kStripes, count);
     TravState s;
     bool has = false;
-    uint32_t sl = 0, n_node = 0, n_tri = 0, n_occ = 0;
+    uint32_t slot = 0, light = 0, n_node = 0, n_tri = 0, n_occ = 0;
     const float4 *nodes = (const float4 *)(B ? bt.nodes : sc0.bvh.nodes);
     const float4 *tris = (const float4 *)(B ? bt.tris : sc0.bvh.tris);
     for (;;) {
@@ -996,9 +1014,25 @@ __global__ __launch_bounds__(kBlock) void k_connect(SceneDev sc0, BatchDev bt, P
         const uint32_t r = wave_claim(c, lcount(q, kLClaimCon, 0), count, has, stripe);
         if (r != 0xffffffffu) {
             const size_t e = stripe * sstride + r;
-            sl = sh.slot[e];
-            const int32_t root = B ? sh.root[e] : 0;
-            trav_begin(s, sh.ox[e], sh.oy[e], sh.oz[e], sh.dx[e], sh.dy[e], sh.dz[e], sh.tmax[e], true, root);
+            const uint32_t ray = sh.ray[e], l = ray & 31u;
+            const size_t vert = (size_t)stripe * q.cs + (ray >> 5);
+            const float4 oa = sh.org[2 * vert], ob = sh.org[2 * vert + 1];
+            const uint32_t sid = bits(ob.w);
+            const SceneDev &sc = B ? bt.scenes[sid] : sc0;
+            const uint32_t npl = sc.npl;
+            slot = bits(ob.z);
+            light = l;
+            V3 w;
+            float tmax;
+            if (l < npl) {
+                V3 tol;
+                w = point_light_dir(sc.pl[l], mk(oa.w, ob.x, ob.y), tol, tmax);
+            } else {
+                const float4 al = sh.area[(size_t)(l - npl) * q.cs * kStripes + vert];
+                w = mk(al.x, al.y, al.z);
+                tmax = al.w;
+            }
+            trav_begin(s, oa.x, oa.y, oa.z, w.x, w.y, w.z, tmax, true, B ? (int32_t)bt.root[sid] : 0);
             has = true;
         }
         if (__ballot(has) == 0) {
@@ -1006,7 +1040,7 @@ __global__ __launch_bounds__(kBlock) void k_connect(SceneDev sc0, BatchDev bt, P
             continue;
         }
         if (has && trav_step_any<WIDE, true, STATS>(s, nodes, tris, stack, cap, leaf_batch(c), n_node, n_tri)) {
-            if (s.occ) atomicAnd(path_word(p, sl >> 5, kPqRng, 3), ~(1u << (sl & 31u)));
+            if (s.occ) atomicAnd(path_word(p, slot, kPqRng, 3), ~(1u << light));
             if (STATS) n_occ += s.occ ? 1u : 0u;
             has = false;
         }

@@ -120,10 +120,16 @@ struct PathsDev {
     float *ttgt;               // compacted targets (P x 3); records compacted into cin
 };
 
+// Shadow rays.  A ray of the list is one word; what it is made of is kept once
+// per shaded vertex, in queue order: the origin and the vertex (k_connect
+// computes a point light's direction and distance again from the vertex,
+// with the operations of the shading), and a sampled area light's direction
+// and distance.  36 bytes per ray written and read back cost a 1080p frame
+// with nine lights 7 of 253 ms.
 struct ShadowDev {
-    float *ox, *oy, *oz, *dx, *dy, *dz, *tmax;
-    uint32_t *slot;             // path slot << 5 | light slot
-    int32_t *root;              // batches: root node of the ray's scene in the pooled tree
+    uint32_t *ray;              // vertex within the stripe << 5 | light slot
+    float4 *org;                // [stripe][vertex]: origin, vertex x | vertex yz, path slot, scene (batches)
+    float4 *area;               // [area light][stripe][vertex]: direction, tMax
 };
 
 struct QueuesDev {

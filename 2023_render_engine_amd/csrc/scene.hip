@@ -348,10 +348,9 @@ rt_status ensure_wave_buffers(WaveBuffers &w, uint32_t P, uint32_t NL, const cha
     add((void **)&p.tB, (size_t)P * 12);
     add((void **)&p.ttgt, (size_t)P * 12);
     ShadowDev &sh = w.shadow;
-    float **sf[] = {&sh.ox, &sh.oy, &sh.oz, &sh.dx, &sh.dy, &sh.dz, &sh.tmax};
-    for (float **f : sf) add((void **)f, SQ * 4);
-    add((void **)&sh.slot, SQ * 4);
-    add((void **)&sh.root, SQ * 4);
+    add((void **)&sh.ray, SQ * 4);
+    add((void **)&sh.org, (size_t)P * 2 * sizeof(float4));
+    add((void **)&sh.area, SQ * sizeof(float4));
     QueuesDev &q = w.queues;
     add((void **)&q.active[0], (size_t)P * 4);
     add((void **)&q.active[1], (size_t)P * 4);
