@@ -22,6 +22,7 @@ struct rt_ctx {
     hipStream_t stream = nullptr;
     std::recursive_mutex lock;
     std::atomic<int> refs{1};
+    rt::BvhBuildSpace bvh_space;   // of rt_bvh_build_device
     void *film_scratch = nullptr;  // partial maxima of the film output kernels, allocated on first use
 };
 
@@ -35,6 +36,7 @@ void ctx_release(rt_ctx *c)
         (void)hipSetDevice(c->device);
         (void)hipStreamSynchronize(c->stream);
         if (c->film_scratch) (void)hipFree(c->film_scratch);
+        c->bvh_space.release();
         (void)hipStreamDestroy(c->stream);
         delete c;
     }
@@ -287,7 +289,6 @@ rt_status rt_bvh_build_device(rt_ctx *ctx, const float *xyz, uint32_t nv, const 
     std::lock_guard<std::recursive_mutex> g(ctx->lock);
     auto drop = [&](rt_status st) {
         rt::free_bvh_device(b->gpu);
-        if (b->ray_counters) (void)hipFree(b->ray_counters);
         delete b;
         return st;
     };
@@ -297,7 +298,8 @@ rt_status rt_bvh_build_device(rt_ctx *ctx, const float *xyz, uint32_t nv, const 
         return drop(RT_ERR_HIP);
     }
     std::string err;
-    he = rt::build_bvh_device(xyz, nv, idx, nt, o, ctx->stream, b->gpu, err);
+    const size_t counters = (size_t)rt_bvh::kRayCounterRing * rt::kClaimWords * sizeof(uint32_t);
+    he = rt::build_bvh_device(xyz, nv, idx, nt, o, ctx->stream, ctx->bvh_space, counters, b->gpu, err);
     if (he != hipSuccess) {
         set_error(err);
         return drop(he == hipErrorInvalidValue ? RT_ERR_INVALID : he == hipErrorOutOfMemory ? RT_ERR_OOM : RT_ERR_HIP);
@@ -316,11 +318,7 @@ rt_status rt_bvh_build_device(rt_ctx *ctx, const float *xyz, uint32_t nv, const 
         set_error("rt_bvh_build_device: tree depth exceeds the traversal stack");
         return drop(RT_ERR_UNSUPPORTED);
     }
-    he = hipMalloc(&b->ray_counters, (size_t)rt_bvh::kRayCounterRing * rt::kClaimWords * sizeof(uint32_t));
-    if (he != hipSuccess) {
-        set_error(std::string("rt_bvh_build_device: ray counters: ") + hipGetErrorString(he));
-        return drop(RT_ERR_OOM);
-    }
+    b->ray_counters = (uint32_t *)d.extra;
     const bool wide = b->width == 4;
     b->dev.nodes = wide ? (void *)d.nodes4 : (void *)d.nodes2;
     b->dev.tris = d.tris;
@@ -352,8 +350,8 @@ rt_status rt_bvh_destroy(rt_bvh *b)
         } else {
             if (b->dev.nodes) (void)hipFree(b->dev.nodes);
             if (b->dev.tris) (void)hipFree(b->dev.tris);
+            if (b->ray_counters) (void)hipFree(b->ray_counters);
         }
-        if (b->ray_counters) (void)hipFree(b->ray_counters);
         if (b->ev0) (void)hipEventDestroy(b->ev0);
         if (b->ev1) (void)hipEventDestroy(b->ev1);
         delete b;

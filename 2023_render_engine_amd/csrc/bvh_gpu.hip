@@ -243,56 +243,187 @@ __device__ inline double area6(const float b[6])
     return 2.0 * (d[0] * d[1] + d[1] * d[2] + d[2] * d[0]);
 }
 
-// Bottom-up boxes and SAH costs in passes: pass p computes every internal
-// node whose children are leaves or were computed in an earlier pass
-// (ready[c] < p).  All it reads was written by earlier launches, so no
-// fence or coherent load is needed; the root is done after as many passes
-// as the tree is high.  Per node: its box (the union of its children's),
-// its SAH cost (cost of a triangle test 1, of a node visit trav_cost, per
-// unit of area) and its choice: a node over at most max_leaf triangles
-// becomes a leaf when (triangles x area) does not exceed (trav_cost x area
-// + its children's costs); and the height of the kept tree below it (0
-// for a node that became a leaf).  The root never becomes a leaf.
-__global__ __launch_bounds__(kBB) void k_node_pass(const uint32_t *child, const uint32_t *lo, const uint32_t *hi,
-                                                   const float *tbox, const uint32_t *val, uint32_t n,
-                                                   uint32_t pass, uint32_t max_leaf, double trav_cost, float *nbox,
-                                                   double *cost, uint32_t *height, uint32_t *leafc, uint32_t *ready)
-{
-    const uint32_t i = blockIdx.x * kBB + threadIdx.x;
-    if (i >= n - 1 || ready[i] != kNotReady) return;
-    const uint32_t c[2] = {child[2 * i], child[2 * i + 1]};
-    for (int k = 0; k < 2; ++k)
-        if (!(c[k] & kLeafBit) && !(ready[c[k]] < pass)) return;
-    float b[2][6];
-    double cc[2];
-    uint32_t hh[2];
-    for (int k = 0; k < 2; ++k) {
-        if (c[k] & kLeafBit) {
-            const float *src = tbox + 6 * (size_t)val[c[k] & ~kLeafBit];
-            for (int j = 0; j < 6; ++j) b[k][j] = src[j];
-            cc[k] = area6(b[k]);
-            hh[k] = 0;
-        } else {
-            for (int j = 0; j < 6; ++j) b[k][j] = nbox[6 * (size_t)c[k] + j];
-            cc[k] = cost[c[k]];
-            hh[k] = height[c[k]];
-        }
-    }
+// A subtree's box, SAH cost and kept height.
+struct NodeVal {
     float box[6];
+    double cost;
+    uint32_t height, leaf;
+};
+
+__device__ inline NodeVal leaf_val(const float *b)
+{
+    NodeVal v;
+    for (int j = 0; j < 6; ++j) v.box[j] = b[j];
+    v.cost = area6(v.box);
+    v.height = 0;
+    v.leaf = 0;
+    return v;
+}
+
+// An internal node from its children: its box (their union), its SAH cost
+// (cost of a triangle test 1, of a node visit trav_cost, per unit of area)
+// and its choice: a node over at most max_leaf triangles becomes a leaf when
+// (triangles x area) does not exceed (trav_cost x area + its children's
+// costs); and the height of the kept tree below it (0 for a node that became
+// a leaf).  The root (i = 0) never becomes a leaf.
+__device__ inline NodeVal node_val(uint32_t i, uint32_t size, const NodeVal &c0, const NodeVal &c1, uint32_t max_leaf,
+                                   double trav_cost)
+{
+    NodeVal v;
     for (int a = 0; a < 3; ++a) {
-        box[a] = fminf(b[0][a], b[1][a]);
-        box[3 + a] = fmaxf(b[0][3 + a], b[1][3 + a]);
+        v.box[a] = fminf(c0.box[a], c1.box[a]);
+        v.box[3 + a] = fmaxf(c0.box[3 + a], c1.box[3 + a]);
     }
-    const double area = area6(box);
-    const double split = trav_cost * area + cc[0] + cc[1];
-    const uint32_t size = hi[i] - lo[i] + 1;
+    const double area = area6(v.box);
+    const double split = trav_cost * area + c0.cost + c1.cost;
     const double as_leaf = (double)size * area;
     const bool leaf = i != 0 && size <= max_leaf && as_leaf <= split;
-    for (int j = 0; j < 6; ++j) nbox[6 * (size_t)i + j] = box[j];
-    cost[i] = leaf ? as_leaf : split;
-    height[i] = leaf ? 0u : 1u + (hh[0] > hh[1] ? hh[0] : hh[1]);
-    leafc[i] = leaf ? 1u : 0u;
-    ready[i] = pass;
+    v.cost = leaf ? as_leaf : split;
+    v.height = leaf ? 0u : 1u + (c0.height > c1.height ? c0.height : c1.height);
+    v.leaf = leaf ? 1u : 0u;
+    return v;
+}
+
+// Bottom-up boxes and SAH costs, in two parts.  A block takes kRun
+// consecutive leaves and every internal node whose range lies inside them (a
+// radix-tree node's own number is one end of its range, so these nodes are
+// numbered within the run), and computes them in LDS, round by round, each
+// node once its children are done.  The nodes whose range crosses the end of a
+// run -- a few thousand above 1M triangles -- go onto a list for k_node_pass.
+// At 2^20 triangles: 63 us here (bound by the reads and writes of ~90 B per
+// triangle) and 24 passes of 4.9 us over the list, launch-bound, in place of
+// 32 passes over every node with a look from the host after each 8.
+constexpr uint32_t kRun = 512;
+struct RunLds {
+    float lbox[kRun][6], nbox[kRun][6];
+    double cost[kRun];
+    uint8_t height[kRun], leaf[kRun], done[kRun];
+    uint32_t ntop, top0;
+};
+
+__global__ __launch_bounds__(kBB) void k_node_runs(const uint32_t *child, const uint32_t *lo, const uint32_t *hi,
+                                                   const float *tbox, const uint32_t *val, uint32_t n,
+                                                   uint32_t max_leaf, double trav_cost, float *nbox, double *cost,
+                                                   uint32_t *height, uint32_t *leafc, uint32_t *ready, uint32_t *top,
+                                                   uint32_t *ntop)
+{
+    __shared__ RunLds r;
+    constexpr uint32_t kPer = kRun / kBB;
+    const uint32_t b0 = blockIdx.x * kRun, b1 = min(b0 + kRun, n);  // leaves [b0, b1)
+    uint32_t c0[kPer], c1[kPer], size[kPer];
+    bool mine[kPer];
+    if (threadIdx.x == 0) r.ntop = 0;
+    for (uint32_t k = 0; k < kPer; ++k) {
+        const uint32_t t = threadIdx.x + k * kBB, i = b0 + t;
+        r.done[t] = 0;
+        mine[k] = false;
+        if (i < b1) {
+            const float *src = tbox + 6 * (size_t)val[i];
+            for (int j = 0; j < 6; ++j) r.lbox[t][j] = src[j];
+        }
+        if (i < n - 1) {
+            const uint32_t l = lo[i], h = hi[i];
+            mine[k] = l >= b0 && h < b1;
+            c0[k] = child[2 * (size_t)i];
+            c1[k] = child[2 * (size_t)i + 1];
+            size[k] = h - l + 1;
+        }
+    }
+    __syncthreads();
+    uint32_t at[kPer];
+    for (uint32_t k = 0; k < kPer; ++k) {
+        const uint32_t i = b0 + threadIdx.x + k * kBB;
+        at[k] = 0;
+        if (i < n - 1 && !mine[k]) at[k] = atomicAdd(&r.ntop, 1u);
+    }
+    auto of = [&](uint32_t c) {
+        const uint32_t t = (c & ~kLeafBit) - b0;
+        if (c & kLeafBit) return leaf_val(r.lbox[t]);
+        NodeVal v;
+        for (int j = 0; j < 6; ++j) v.box[j] = r.nbox[t][j];
+        v.cost = r.cost[t];
+        v.height = r.height[t];
+        v.leaf = r.leaf[t];
+        return v;
+    };
+    auto is_done = [&](uint32_t c) { return (c & kLeafBit) || r.done[(c & ~kLeafBit) - b0]; };
+    bool left[kPer];
+    for (uint32_t k = 0; k < kPer; ++k) left[k] = mine[k];
+    for (;;) {
+        // every turn finishes at least the lowest nodes left, so the loop ends
+        bool now[kPer], any = false;
+        for (uint32_t k = 0; k < kPer; ++k) {
+            now[k] = left[k] && is_done(c0[k]) && is_done(c1[k]);
+            any = any || left[k];
+        }
+        if (!__syncthreads_or(any)) break;
+        for (uint32_t k = 0; k < kPer; ++k) {
+            if (!now[k]) continue;
+            const uint32_t t = threadIdx.x + k * kBB;
+            const NodeVal v = node_val(b0 + t, size[k], of(c0[k]), of(c1[k]), max_leaf, trav_cost);
+            for (int j = 0; j < 6; ++j) r.nbox[t][j] = v.box[j];
+            r.cost[t] = v.cost;
+            r.height[t] = (uint8_t)v.height;
+            r.leaf[t] = (uint8_t)v.leaf;
+            left[k] = false;
+        }
+        __syncthreads();
+        for (uint32_t k = 0; k < kPer; ++k)
+            if (now[k]) r.done[threadIdx.x + k * kBB] = 1;
+        __syncthreads();
+    }
+    if (threadIdx.x == 0) r.top0 = r.ntop ? atomicAdd(ntop, r.ntop) : 0u;
+    __syncthreads();
+    for (uint32_t k = 0; k < kPer; ++k) {
+        const uint32_t t = threadIdx.x + k * kBB, i = b0 + t;
+        if (i >= n - 1) continue;
+        if (mine[k]) {
+            for (int j = 0; j < 6; ++j) nbox[6 * (size_t)i + j] = r.nbox[t][j];
+            cost[i] = r.cost[t];
+            height[i] = r.height[t];
+            leafc[i] = r.leaf[t];
+            ready[i] = 0;
+        } else {
+            ready[i] = kNotReady;
+            top[r.top0 + at[k]] = i;
+        }
+    }
+}
+
+// The nodes of the list, in passes: pass p computes every one whose children
+// are leaves or were computed earlier (ready[c] < p).  All it reads was
+// written by earlier launches, so no fence or coherent load is needed.
+__global__ __launch_bounds__(kBB) void k_node_pass(const uint32_t *child, const uint32_t *lo, const uint32_t *hi,
+                                                   const float *tbox, const uint32_t *val, const uint32_t *top,
+                                                   const uint32_t *ntop, uint32_t pass, uint32_t max_leaf,
+                                                   double trav_cost, float *nbox, double *cost, uint32_t *height,
+                                                   uint32_t *leafc, uint32_t *ready)
+{
+    const uint32_t m = *ntop;
+    for (uint32_t t = blockIdx.x * kBB + threadIdx.x; t < m; t += gridDim.x * kBB) {
+        const uint32_t i = top[t];
+        if (ready[i] != kNotReady) continue;
+        const uint32_t c[2] = {child[2 * (size_t)i], child[2 * (size_t)i + 1]};
+        bool ok = true;
+        for (int k = 0; k < 2; ++k)
+            if (!(c[k] & kLeafBit) && !(ready[c[k]] < pass)) ok = false;
+        if (!ok) continue;
+        auto of = [&](uint32_t ch) {
+            if (ch & kLeafBit) return leaf_val(tbox + 6 * (size_t)val[ch & ~kLeafBit]);
+            NodeVal v;
+            for (int j = 0; j < 6; ++j) v.box[j] = nbox[6 * (size_t)ch + j];
+            v.cost = cost[ch];
+            v.height = height[ch];
+            v.leaf = leafc[ch];
+            return v;
+        };
+        const NodeVal v = node_val(i, hi[i] - lo[i] + 1, of(c[0]), of(c[1]), max_leaf, trav_cost);
+        for (int j = 0; j < 6; ++j) nbox[6 * (size_t)i + j] = v.box[j];
+        cost[i] = v.cost;
+        height[i] = v.height;
+        leafc[i] = v.leaf;
+        ready[i] = pass;
+    }
 }
 
 // Kept internal nodes: the root, and every node neither of whose own
@@ -325,10 +456,10 @@ __global__ __launch_bounds__(kBB) void k_emit_node2(const uint32_t *child, const
                                                     const uint32_t *cb, Node2 *nodes, double *sah)
 {
     __shared__ double part[kBB];
-    const uint32_t i = blockIdx.x * kBB + threadIdx.x;
     double acc = 0.0;
-    if (i < n - 1 && keep[i]) {
-        const float pad = scene_pad(cb);
+    const float pad = scene_pad(cb);
+    for (uint32_t i = blockIdx.x * kBB + threadIdx.x; i < n - 1; i += gridDim.x * kBB) {
+        if (!keep[i]) continue;
         Node2 nd{};
         float bx[2][6];
         for (int c = 0; c < 2; ++c) {
@@ -413,15 +544,14 @@ __device__ inline void node2_kids(const Node2 &n, Kid &k0, Kid &k1)
     k1.ref = n.child[1];
 }
 
-// Smallest power-of-two scale 2^e (e >= -126) with 255 * 2^e >= extent.
+// Smallest e >= -126 with 255 * 2^e >= extent: with extent = m * 2^k, m in
+// [0.5, 1), 2^(k - 8) is enough up to m = 255/256 and 2^(k - 9) never is.
 __device__ inline int scale_exponent(double extent)
 {
     if (!(extent > 0.0)) return -126;
-    int e = (int)ceil(log2(extent / 255.0));
-    if (e < -126) e = -126;
-    while (255.0 * ldexp(1.0, e) < extent) ++e;
-    while (e > -126 && 255.0 * ldexp(1.0, e - 1) >= extent) --e;
-    return e;
+    int k;
+    const double m = frexp(extent, &k);
+    return max(-126, k - 8 + (m > 255.0 / 256.0 ? 1 : 0));
 }
 
 // The kids of a wide node: its two-wide node's two children, then the
@@ -448,39 +578,108 @@ __device__ inline int open_kids(const Node2 *n2, uint32_t src, Kid kids[4])
     return nk;
 }
 
-// One level, first pass: internal kids per frontier entry.
-__global__ __launch_bounds__(kBB) void k_collapse4_count(const Node2 *n2, const uint2 *front, uint32_t nfront,
-                                                         uint32_t *cnt)
+// The collapse's levels.  A level's figures are written on the device by the
+// level before it, so the levels are launched one after the other without a
+// look from the host; levels past the last find nothing to do.  At 2^20
+// triangles (12 levels) this takes 0.42 ms, where a scan's launches, two
+// copies and a wait per level took 1.3; the small levels are launch-bound
+// (4-5 us each), the large ones wait on the gathers of two-wide nodes.
+struct Level {
+    uint32_t nfront, base;  // frontier entries, and the first one's wide node
+};
+
+// The frontier entries of a block of a level: contiguous, whole tiles.
+__device__ inline void level_share(uint32_t nfront, uint32_t &f0, uint32_t &f1)
 {
-    const uint32_t f = blockIdx.x * kBB + threadIdx.x;
-    if (f >= nfront) return;
-    Kid kids[4];
-    const int nk = open_kids(n2, front[f].x, kids);
-    uint32_t ni = 0;
-    for (int i = 0; i < nk; ++i) ni += kids[i].ref >= 0 ? 1u : 0u;
-    cnt[f] = ni;
+    const uint32_t tiles = (nfront + kBB - 1) / kBB, per = (tiles + gridDim.x - 1) / gridDim.x;
+    f0 = min(blockIdx.x * per * kBB, nfront);
+    f1 = min(f0 + per * kBB, nfront);
 }
 
-// One level, second pass: frontier entry f (two-wide node, pending entries
-// above it) becomes wide node base + f; its internal kids, in slot order,
-// become next-level entries off[f], off[f] + 1, ... and wide nodes
-// base + nfront + off[f] + j.  The numbering is breadth-first and does not
-// depend on scheduling.  The four-wide traversal holds at most
-// (pending above) + kids - 1 entries at a node, so the deepest such sum is
-// its stack bound (*need), the host collapse's figure.
-__global__ __launch_bounds__(kBB) void k_collapse4(const Node2 *n2, const uint2 *front, uint32_t nfront,
-                                                   const uint32_t *off, uint32_t base, uint32_t sentinel, Node4 *n4,
-                                                   uint2 *next, uint32_t *need)
+// One level, first pass: internal kids per frontier entry and per block.
+__global__ __launch_bounds__(kBB) void k_collapse4_count(const Node2 *n2, const uint2 *front, const Level *level,
+                                                         uint32_t *cnt, uint32_t *bsum)
 {
-    const uint32_t f = blockIdx.x * kBB + threadIdx.x;
-    if (f >= nfront) return;
+    __shared__ uint32_t red[kBB];
+    uint32_t f0, f1, sum = 0;
+    level_share(level->nfront, f0, f1);
+    for (uint32_t f = f0 + threadIdx.x; f < f1; f += kBB) {
+        Kid kids[4];
+        const int nk = open_kids(n2, front[f].x, kids);
+        uint32_t ni = 0;
+        for (int i = 0; i < nk; ++i) ni += kids[i].ref >= 0 ? 1u : 0u;
+        cnt[f] = ni;
+        sum += ni;
+    }
+    red[threadIdx.x] = sum;
+    __syncthreads();
+    for (int s = kBB / 2; s > 0; s >>= 1) {
+        if ((int)threadIdx.x < s) red[threadIdx.x] += red[threadIdx.x + s];
+        __syncthreads();
+    }
+    if (threadIdx.x == 0) bsum[blockIdx.x] = red[0];
+}
+
+__device__ void collapse_entry(const Node2 *n2, const uint2 *front, uint32_t f, uint32_t nfront, uint32_t q,
+                               uint32_t base, uint32_t sentinel, Node4 *n4, uint2 *next, uint32_t &need);
+
+// One level, second pass: the entries' offsets from the blocks' sums and a
+// prefix sum per tile; the last block writes the next level's figures.
+__global__ __launch_bounds__(kBB) void k_collapse4(const Node2 *n2, const uint2 *front, Level *level,
+                                                   const uint32_t *cnt, const uint32_t *bsum, uint32_t sentinel,
+                                                   Node4 *n4, uint2 *next, uint32_t *need)
+{
+    __shared__ uint32_t sc[kBB];
+    const Level lv = *level;
+    uint32_t before = 0;
+    for (uint32_t b = threadIdx.x; b < blockIdx.x; b += kBB) before += bsum[b];
+    sc[threadIdx.x] = before;
+    __syncthreads();
+    for (int s = kBB / 2; s > 0; s >>= 1) {
+        if ((int)threadIdx.x < s) sc[threadIdx.x] += sc[threadIdx.x + s];
+        __syncthreads();
+    }
+    uint32_t off = sc[0], most = 0;
+    if (blockIdx.x == gridDim.x - 1 && threadIdx.x == 0) {
+        level[1].nfront = off + bsum[blockIdx.x];
+        level[1].base = lv.base + lv.nfront;
+    }
+    uint32_t f0, f1;
+    level_share(lv.nfront, f0, f1);
+    for (uint32_t t0 = f0; t0 < f1; t0 += kBB) {
+        const uint32_t f = t0 + threadIdx.x;
+        const uint32_t mine = f < f1 ? cnt[f] : 0u;
+        __syncthreads();
+        sc[threadIdx.x] = mine;
+        __syncthreads();
+        for (int s = 1; s < kBB; s <<= 1) {
+            const uint32_t v = (int)threadIdx.x >= s ? sc[threadIdx.x - s] : 0u;
+            __syncthreads();
+            sc[threadIdx.x] += v;
+            __syncthreads();
+        }
+        if (f < f1) collapse_entry(n2, front, f, lv.nfront, off + sc[threadIdx.x] - mine, lv.base, sentinel, n4, next, most);
+        off += sc[kBB - 1];
+    }
+    for (int o = 32; o > 0; o >>= 1) most = max(most, (uint32_t)__shfl_xor((int)most, o));
+    if ((threadIdx.x & 63u) == 0 && most) atomicMax(need, most);
+}
+
+// Frontier entry f (two-wide node, pending entries above it) becomes wide
+// node base + f; its internal kids, in slot order, become next-level entries
+// q, q + 1, ... and wide nodes base + nfront + q + j.  The numbering is
+// breadth-first and does not depend on scheduling.  The four-wide traversal
+// holds at most (pending above) + kids - 1 entries at a node, so the deepest
+// such sum is its stack bound (need), the host collapse's figure.
+__device__ void collapse_entry(const Node2 *n2, const uint2 *front, uint32_t f, uint32_t nfront, uint32_t q,
+                               uint32_t base, uint32_t sentinel, Node4 *n4, uint2 *next, uint32_t &need)
+{
     const uint2 fe = front[f];
     Kid kids[4];
     const int nk = open_kids(n2, fe.x, kids);
     const uint32_t pending = fe.y + (uint32_t)nk - 1u;
-    atomicMax(need, pending);
+    need = max(need, pending);
     int32_t refs[4];
-    uint32_t q = off[f];
     for (int i = 0; i < nk; ++i) {
         if (kids[i].ref >= 0) {
             next[q] = make_uint2((uint32_t)kids[i].ref, pending);
@@ -499,13 +698,13 @@ __global__ __launch_bounds__(kBB) void k_collapse4(const Node2 *n2, const uint2 
         double ext = 0.0;
         for (int i = 0; i < nk; ++i) ext = fmax(ext, (double)kids[i].hi[a] - (double)p);
         const int e = scale_exponent(ext);
-        const double sc = ldexp(1.0, e);
+        const double sc = ldexp(1.0, e), inv = ldexp(1.0, -e);  // x * inv is x / sc exactly
         n.origin[a] = p;
         meta |= (uint32_t)(e + 127) << (8 * a);
         uint32_t qlo = 0, qhi = 0;
         for (int i = 0; i < nk; ++i) {
-            double l = floor(((double)kids[i].lo[a] - (double)p) / sc);
-            double h = ceil(((double)kids[i].hi[a] - (double)p) / sc);
+            double l = floor(((double)kids[i].lo[a] - (double)p) * inv);
+            double h = ceil(((double)kids[i].hi[a] - (double)p) * inv);
             l = fmin(fmax(l, 0.0), 255.0);
             h = fmin(fmax(h, 0.0), 255.0);
             while (l > 0.0 && (double)p + l * sc > (double)kids[i].lo[a]) l -= 1.0;
@@ -523,17 +722,56 @@ __global__ __launch_bounds__(kBB) void k_collapse4(const Node2 *n2, const uint2 
     n4[base + f] = n;
 }
 
-unsigned blocks(uint64_t n) { return (unsigned)std::max<uint64_t>(1, (n + kBB - 1) / kBB); }
-
-struct Arena {
-    char *base = nullptr;
-    ~Arena() { if (base) (void)hipFree(base); }
+// What the host reads back from a build: gathered, so that it is one copy.
+struct BuildInfo {
+    uint32_t nodes, bad, height;
+    float root_box[6];
 };
+
+__global__ void k_build_info(const uint32_t *last_idx, const uint32_t *last_keep, const uint32_t *bad,
+                             const uint32_t *height, const float *nbox, BuildInfo *out)
+{
+    if (threadIdx.x != 0) return;
+    BuildInfo in;
+    in.nodes = *last_idx + *last_keep;
+    in.bad = *bad;
+    in.height = *height;
+    for (int j = 0; j < 6; ++j) in.root_box[j] = nbox[j];
+    *out = in;
+}
+
+constexpr uint32_t kLevels = 16, kMaxLevels = 64;
+constexpr unsigned kCollapseBlocks = 512;
+constexpr unsigned kEmitBlocks = 1024;  // each ends in one atomic on the SAH sum
+struct CollapseState {
+    Level level[kMaxLevels + 1];
+    uint32_t need;
+};
+
+// The root's frontier entry and the level table's start.
+__global__ void k_collapse4_begin(uint2 *front, CollapseState *st)
+{
+    for (uint32_t l = threadIdx.x; l <= kMaxLevels; l += blockDim.x) st->level[l] = Level{l == 0 ? 1u : 0u, 0u};
+    if (threadIdx.x == 0) {
+        front[0] = make_uint2(0u, 0u);
+        st->need = 0;
+    }
+}
+
+struct BuildReadback {
+    uint32_t root_ready;
+    BuildInfo info;
+    double sah;
+    CollapseState collapse;
+};
+static_assert(sizeof(BuildReadback) <= BvhBuildSpace::kPinned, "the pinned block holds every read-back");
+
+unsigned blocks(uint64_t n) { return (unsigned)std::max<uint64_t>(1, (n + kBB - 1) / kBB); }
 
 }  // namespace
 
 hipError_t build_bvh_device(const float *xyz, uint32_t nv, const uint32_t *idx, uint32_t nt, const rt_bvh_opts &o,
-                            hipStream_t s, DeviceBvhBuild &out, std::string &err)
+                            hipStream_t s, BvhBuildSpace &space, size_t extra, DeviceBvhBuild &out, std::string &err)
 {
     const auto t0 = std::chrono::steady_clock::now();
     out = DeviceBvhBuild{};
@@ -544,11 +782,30 @@ hipError_t build_bvh_device(const float *xyz, uint32_t nv, const uint32_t *idx, 
         err = std::string("rt_bvh_build_device: ") + what + ": " + hipGetErrorString(x);
         return x;
     };
-    // outputs: two-wide nodes (at least one), triangles + sentinel
-    const uint32_t n2_cap = nt > 1 ? nt - 1 : 1;
-    if ((e = hipMalloc(&out.nodes2, (size_t)n2_cap * sizeof(Node2))) != hipSuccess) return fail(e, "nodes");
-    if ((e = hipMalloc(&out.tris, ((size_t)nt + 1) * sizeof(Tri3))) != hipSuccess) return fail(e, "triangles");
+    // outputs: `nodes` two-wide nodes, as many wide nodes (each takes at least
+    // one two-wide node of its own), triangles + sentinel and the caller's
+    // `extra` bytes, in one allocation
+    auto allocate = [&](uint32_t nodes) {
+        const size_t o4 = (size_t)nodes * sizeof(Node2), ot = o4 + (wide ? (size_t)nodes * sizeof(Node4) : 0);
+        const size_t ox = (ot + ((size_t)nt + 1) * sizeof(Tri3) + 255) & ~(size_t)255;
+        char *m = nullptr;
+        const hipError_t x = hipMalloc(&m, ox + extra);
+        if (x != hipSuccess) return x;
+        out.nodes2 = (Node2 *)m;
+        out.nodes4 = wide ? (Node4 *)(m + o4) : nullptr;
+        out.tris = (Tri3 *)(m + ot);
+        out.extra = m + ox;
+        return x;
+    };
+    struct Trim {
+        BvhBuildSpace &space;
+        hipStream_t s;
+        ~Trim() { space.trim(s); }
+    } trim{space, s};
     out.num_tris = nt;
+    if ((e = space.reserve_pinned()) != hipSuccess) return fail(e, "pinned read-back");
+    BuildReadback &rb = *(BuildReadback *)space.pinned;
+    rb = BuildReadback{};
     if (nt <= 1) {
         // one node on the host: the triangle (if any) and the sentinel
         std::vector<float> v(9, 0.0f);
@@ -589,6 +846,7 @@ hipError_t build_bvh_device(const float *xyz, uint32_t nv, const uint32_t *idx, 
         root.f[0] = lo[0]; root.f[1] = hi[0]; root.f[2] = lo[1]; root.f[3] = hi[1]; root.f[8] = lo[2]; root.f[9] = hi[2];
         root.child[0] = encode_leaf(nt ? 0u : nt, 1);
         root.child[1] = encode_leaf(nt, 1);
+        if ((e = allocate(1)) != hipSuccess) return fail(e, "tree");
         if ((e = hipMemcpyAsync(out.nodes2, &root, sizeof root, hipMemcpyHostToDevice, s)) != hipSuccess ||
             (e = hipMemcpyAsync(out.tris, tr + (nt ? 0 : 1), (nt + 1) * sizeof(Tri3), hipMemcpyHostToDevice, s)) !=
                 hipSuccess ||
@@ -607,7 +865,7 @@ hipError_t build_bvh_device(const float *xyz, uint32_t nv, const uint32_t *idx, 
                      o_key2 = take(N * 4), o_val = take(N * 4), o_val2 = take(N * 4), o_child = take(2 * N * 4),
                      o_lo = take(N * 4), o_hi = take(N * 4), o_parent = take(2 * N * 4), o_nbox = take(N * 24),
                      o_cost = take(N * 8), o_height = take(N * 4), o_leafc = take(N * 4), o_ready = take(N * 4),
-                     o_keep = take(N * 4), o_new = take(N * 4);
+                     o_keep = take(N * 4), o_new = take(N * 4), o_top = take(N * 4);
         size_t sort_bytes = 0, scan_bytes = 0;
         if ((e = hipcub::DeviceRadixSort::SortPairs(nullptr, sort_bytes, (const uint32_t *)nullptr, (uint32_t *)nullptr,
                                                     (const uint32_t *)nullptr, (uint32_t *)nullptr, (int)N, 0, 30, s)) !=
@@ -616,22 +874,19 @@ hipError_t build_bvh_device(const float *xyz, uint32_t nv, const uint32_t *idx, 
                                                   (int)(N - 1), s)) != hipSuccess)
             return fail(e, "sizing");
         const size_t o_tmp = take(std::max(sort_bytes, scan_bytes));
-        Arena ar;
-        if ((e = hipMalloc(&ar.base, off)) != hipSuccess) return fail(e, "work space");
-        char *b = ar.base;
+        if ((e = space.reserve(off, s)) != hipSuccess) return fail(e, "work space");
+        char *b = (char *)space.dev;
         float *tbox = (float *)(b + o_tbox), *nbox = (float *)(b + o_nbox);
         // cb: centre and box bounds (12 words), the bad-input flag, then the
-        // SAH sum (a double at word 14)
-        uint32_t *cb = (uint32_t *)(b + o_cb), *bad = cb + 12;
+        // SAH sum (a double at word 14); word 13 the length of the top list
+        uint32_t *cb = (uint32_t *)(b + o_cb), *bad = cb + 12, *ntop = cb + 13, *top = (uint32_t *)(b + o_top);
         double *sah = (double *)(cb + 14), *cost = (double *)(b + o_cost);
         uint32_t *part = (uint32_t *)(b + o_part), *key = (uint32_t *)(b + o_key), *key2 = (uint32_t *)(b + o_key2),
                  *val = (uint32_t *)(b + o_val), *val2 = (uint32_t *)(b + o_val2), *child = (uint32_t *)(b + o_child),
                  *lo = (uint32_t *)(b + o_lo), *hi = (uint32_t *)(b + o_hi), *parent = (uint32_t *)(b + o_parent),
                  *height = (uint32_t *)(b + o_height), *leafc = (uint32_t *)(b + o_leafc),
                  *ready = (uint32_t *)(b + o_ready), *keep = (uint32_t *)(b + o_keep), *newidx = (uint32_t *)(b + o_new);
-        if ((e = hipMemsetAsync(cb, 0, 16 * 4, s)) != hipSuccess ||
-            (e = hipMemsetAsync(ready, 0xff, N * 4, s)) != hipSuccess)
-            return fail(e, "clear");
+        if ((e = hipMemsetAsync(cb, 0, 16 * 4, s)) != hipSuccess) return fail(e, "clear");
         const double trav_cost = o.trav_cost > 0 ? o.trav_cost : 1.2f;
         hipLaunchKernelGGL(k_tri_boxes, dim3(nb), dim3(kBB), 0, s, xyz, nv, idx, nt, tbox, part, bad);
         hipLaunchKernelGGL(k_bounds, dim3(1), dim3(kBB), 0, s, part, (uint32_t)nb, cb);
@@ -642,21 +897,25 @@ hipError_t build_bvh_device(const float *xyz, uint32_t nv, const uint32_t *idx, 
             return fail(e, "sort");
         hipLaunchKernelGGL(k_radix_tree, dim3(blocks(N - 1)), dim3(kBB), 0, s, key2, nt, child, lo, hi, parent);
         if ((e = hipGetLastError()) != hipSuccess) return fail(e, "radix tree");
-        // passes in batches of eight until the root is done; a radix tree of
-        // 30-bit codes split further by 32-bit positions is at most 62 high
-        uint32_t pass = 0, root_ready = kNotReady;
-        while (root_ready == kNotReady) {
+        hipLaunchKernelGGL(k_node_runs, dim3((unsigned)((N + kRun - 1) / kRun)), dim3(kBB), 0, s, child, lo, hi, tbox,
+                           val2, nt, max_leaf, trav_cost, nbox, cost, height, leafc, ready, top, ntop);
+        // passes over the rest until the root is done: its `ready` word is read
+        // back after 24 and then every 8 (a look costs as much as 6 passes).  A radix tree of 30-bit codes split further by 32-bit positions
+        // is at most 62 high
+        uint32_t pass = 0;
+        rb.root_ready = nt > kRun ? kNotReady : 0u;
+        while (rb.root_ready == kNotReady) {
             if (pass >= 64) {
                 err = "rt_bvh_build_device: radix tree higher than 64 levels";
                 return hipErrorUnknown;
             }
-            for (int k = 0; k < 8; ++k) {
+            for (int k = pass ? 8 : 24; k > 0; --k) {
                 ++pass;
-                hipLaunchKernelGGL(k_node_pass, dim3(blocks(N - 1)), dim3(kBB), 0, s, child, lo, hi, tbox, val2, nt,
-                                   pass, max_leaf, trav_cost, nbox, cost, height, leafc, ready);
+                hipLaunchKernelGGL(k_node_pass, dim3(std::min(blocks(N), 64u)), dim3(kBB), 0, s, child, lo, hi, tbox,
+                                   val2, top, ntop, pass, max_leaf, trav_cost, nbox, cost, height, leafc, ready);
             }
             if ((e = hipGetLastError()) != hipSuccess ||
-                (e = hipMemcpyAsync(&root_ready, ready, 4, hipMemcpyDeviceToHost, s)) != hipSuccess ||
+                (e = hipMemcpyAsync(&rb.root_ready, ready, 4, hipMemcpyDeviceToHost, s)) != hipSuccess ||
                 (e = hipStreamSynchronize(s)) != hipSuccess)
                 return fail(e, "boxes");
         }
@@ -664,85 +923,75 @@ hipError_t build_bvh_device(const float *xyz, uint32_t nv, const uint32_t *idx, 
         if ((e = hipGetLastError()) != hipSuccess) return fail(e, "collapse");
         if ((e = hipcub::DeviceScan::ExclusiveSum(b + o_tmp, scan_bytes, keep, newidx, (int)(N - 1), s)) != hipSuccess)
             return fail(e, "scan");
-        hipLaunchKernelGGL(k_emit_node2, dim3(blocks(N - 1)), dim3(kBB), 0, s, child, lo, hi, keep, newidx, tbox, val2,
-                           nbox, nt, cb, out.nodes2, sah);
-        hipLaunchKernelGGL(k_emit_tris, dim3(blocks(N + 1)), dim3(kBB), 0, s, xyz, nv, idx, val2, nt, out.tris);
-        if ((e = hipGetLastError()) != hipSuccess) return fail(e, "emit");
-        uint32_t last[2] = {0, 0}, bad_h = 0, height_h = 0;
-        double sah_h = 0.0;
-        float root_box[6];
-        if ((e = hipMemcpyAsync(last, newidx + (N - 2), 4, hipMemcpyDeviceToHost, s)) != hipSuccess ||
-            (e = hipMemcpyAsync(last + 1, keep + (N - 2), 4, hipMemcpyDeviceToHost, s)) != hipSuccess ||
-            (e = hipMemcpyAsync(&bad_h, bad, 4, hipMemcpyDeviceToHost, s)) != hipSuccess ||
-            (e = hipMemcpyAsync(&height_h, height, 4, hipMemcpyDeviceToHost, s)) != hipSuccess ||
-            (e = hipMemcpyAsync(&sah_h, sah, 8, hipMemcpyDeviceToHost, s)) != hipSuccess ||
-            (e = hipMemcpyAsync(root_box, nbox, 24, hipMemcpyDeviceToHost, s)) != hipSuccess ||
+        hipLaunchKernelGGL(k_build_info, dim3(1), dim3(64), 0, s, newidx + (N - 2), keep + (N - 2), bad, height, nbox,
+                           (BuildInfo *)(b + o_part));
+        if ((e = hipGetLastError()) != hipSuccess ||
+            (e = hipMemcpyAsync(&rb.info, b + o_part, sizeof(BuildInfo), hipMemcpyDeviceToHost, s)) != hipSuccess ||
             (e = hipStreamSynchronize(s)) != hipSuccess)
             return fail(e, "read-back");
-        if (bad_h) { err = "rt_bvh_build_device: triangle index out of range or non-finite coordinate"; return hipErrorInvalidValue; }
-        out.num_nodes2 = last[0] + last[1];
-        out.max_depth = height_h;
-        double ra = 0.0;
-        {
-            double d[3];
-            for (int a = 0; a < 3; ++a) d[a] = std::max(0.0, (double)root_box[3 + a] - (double)root_box[a]);
-            ra = 2.0 * (d[0] * d[1] + d[1] * d[2] + d[2] * d[0]);
-        }
-        out.sah_cost = ra > 0 ? sah_h / ra : 0.0;
+        const BuildInfo &in = rb.info;
+        if (in.bad) { err = "rt_bvh_build_device: triangle index out of range or non-finite coordinate"; return hipErrorInvalidValue; }
+        out.num_nodes2 = in.nodes;
+        out.max_depth = in.height;
+        if ((e = allocate(in.nodes)) != hipSuccess) return fail(e, "tree");
+        hipLaunchKernelGGL(k_emit_node2, dim3(std::min(blocks(N - 1), kEmitBlocks)), dim3(kBB), 0, s, child, lo, hi, keep, newidx, tbox, val2,
+                           nbox, nt, cb, out.nodes2, sah);
+        hipLaunchKernelGGL(k_emit_tris, dim3(blocks(N + 1)), dim3(kBB), 0, s, xyz, nv, idx, val2, nt, out.tris);
+        if ((e = hipGetLastError()) != hipSuccess ||
+            (e = hipMemcpyAsync(&rb.sah, sah, 8, hipMemcpyDeviceToHost, s)) != hipSuccess)
+            return fail(e, "emit");
         // a binary tree of m kept nodes has m + 1 leaves
         out.num_leaves = out.num_nodes2 + 1;
     }
     if (wide) {
-        // level by level from the root, breadth-first numbering.  Each wide
-        // node takes at least one two-wide node of its own, so num_nodes2
-        // bounds both the wide nodes and any level's frontier.
+        // level by level from the root, breadth-first numbering, kLevels of them
+        // (each is two launches) before a look at how far it went; num_nodes2
+        // bounds any level's frontier
         const uint32_t cap4 = out.num_nodes2;
-        if ((e = hipMalloc(&out.nodes4, (size_t)cap4 * sizeof(Node4))) != hipSuccess) return fail(e, "wide nodes");
-        size_t scan_bytes = 0;
-        if ((e = hipcub::DeviceScan::ExclusiveSum(nullptr, scan_bytes, (const uint32_t *)nullptr, (uint32_t *)nullptr,
-                                                  (int)cap4, s)) != hipSuccess)
-            return fail(e, "sizing");
+        const unsigned grid = std::min(blocks(cap4), kCollapseBlocks);
         size_t off = 0;
         auto take = [&](size_t bytes) { size_t r = off; off += (bytes + 255) & ~(size_t)255; return r; };
+        // (the build's own arrays are not read any more)
         const size_t o_f0 = take((size_t)cap4 * 8), o_f1 = take((size_t)cap4 * 8), o_cnt = take((size_t)cap4 * 4),
-                     o_off = take((size_t)cap4 * 4), o_need = take(4), o_tmp = take(scan_bytes);
-        Arena fr;
-        if ((e = hipMalloc(&fr.base, off)) != hipSuccess) return fail(e, "frontier");
-        uint2 *front[2] = {(uint2 *)(fr.base + o_f0), (uint2 *)(fr.base + o_f1)};
-        uint32_t *cnt = (uint32_t *)(fr.base + o_cnt), *offs = (uint32_t *)(fr.base + o_off),
-                 *need = (uint32_t *)(fr.base + o_need);
-        const uint2 root = make_uint2(0u, 0u);
-        if ((e = hipMemcpyAsync(front[0], &root, sizeof root, hipMemcpyHostToDevice, s)) != hipSuccess ||
-            (e = hipMemsetAsync(need, 0, 4, s)) != hipSuccess)
-            return fail(e, "frontier");
-        uint32_t nfront = 1, level = 0, base = 0;
-        while (nfront) {
-            const uint32_t cur = level & 1u;
-            hipLaunchKernelGGL(k_collapse4_count, dim3(blocks(nfront)), dim3(kBB), 0, s, out.nodes2, front[cur], nfront,
-                               cnt);
+                     o_bsum = take(kCollapseBlocks * 4), o_lev = take(sizeof(CollapseState));
+        if ((e = space.reserve(off, s)) != hipSuccess) return fail(e, "frontier");
+        char *b = (char *)space.dev;
+        uint2 *front[2] = {(uint2 *)(b + o_f0), (uint2 *)(b + o_f1)};
+        uint32_t *cnt = (uint32_t *)(b + o_cnt), *bsum = (uint32_t *)(b + o_bsum);
+        CollapseState *st = (CollapseState *)(b + o_lev);
+        hipLaunchKernelGGL(k_collapse4_begin, dim3(1), dim3(64), 0, s, front[0], st);
+        uint32_t level = 0;
+        for (bool more = true; more;) {
+            if (level + kLevels > kMaxLevels) {
+                err = "rt_bvh_build_device: four-wide tree deeper than its two-wide tree can be";
+                return hipErrorUnknown;
+            }
+            for (uint32_t k = 0; k < kLevels; ++k, ++level) {
+                const uint32_t cur = level & 1u;
+                hipLaunchKernelGGL(k_collapse4_count, dim3(grid), dim3(kBB), 0, s, out.nodes2, front[cur],
+                                   st->level + level, cnt, bsum);
+                hipLaunchKernelGGL(k_collapse4, dim3(grid), dim3(kBB), 0, s, out.nodes2, front[cur], st->level + level,
+                                   cnt, bsum, out.num_tris, out.nodes4, front[cur ^ 1u], &st->need);
+            }
             if ((e = hipGetLastError()) != hipSuccess ||
-                (e = hipcub::DeviceScan::ExclusiveSum(fr.base + o_tmp, scan_bytes, cnt, offs, (int)nfront, s)) !=
-                    hipSuccess)
-                return fail(e, "collapse");
-            hipLaunchKernelGGL(k_collapse4, dim3(blocks(nfront)), dim3(kBB), 0, s, out.nodes2, front[cur], nfront,
-                               offs, base, out.num_tris, out.nodes4, front[cur ^ 1u], need);
-            uint32_t tail[2] = {0, 0};
-            if ((e = hipGetLastError()) != hipSuccess ||
-                (e = hipMemcpyAsync(tail, offs + nfront - 1, 4, hipMemcpyDeviceToHost, s)) != hipSuccess ||
-                (e = hipMemcpyAsync(tail + 1, cnt + nfront - 1, 4, hipMemcpyDeviceToHost, s)) != hipSuccess ||
+                (e = hipMemcpyAsync(&rb.collapse, st, sizeof(CollapseState), hipMemcpyDeviceToHost, s)) != hipSuccess ||
                 (e = hipStreamSynchronize(s)) != hipSuccess)
                 return fail(e, "collapse");
-            base += nfront;
-            nfront = tail[0] + tail[1];
-            ++level;
+            more = rb.collapse.level[level].nfront != 0;
         }
-        uint32_t need_h = 0;
-        if ((e = hipMemcpyAsync(&need_h, need, 4, hipMemcpyDeviceToHost, s)) != hipSuccess ||
-            (e = hipStreamSynchronize(s)) != hipSuccess)
-            return fail(e, "collapse");
-        out.num_nodes4 = base;
-        out.depth4 = level;
-        out.max_stack4 = need_h;
+        uint32_t depth = 0;
+        while (depth < level && rb.collapse.level[depth].nfront != 0) ++depth;
+        out.num_nodes4 = rb.collapse.level[depth].base;
+        out.depth4 = depth;
+        out.max_stack4 = rb.collapse.need;
+    }
+    if (!wide && (e = hipStreamSynchronize(s)) != hipSuccess) return fail(e, "emit");
+    if (nt > 1) {
+        double d[3];
+        for (int a = 0; a < 3; ++a)
+            d[a] = std::max(0.0, (double)rb.info.root_box[3 + a] - (double)rb.info.root_box[a]);
+        const double ra = 2.0 * (d[0] * d[1] + d[1] * d[2] + d[2] * d[0]);
+        out.sah_cost = ra > 0 ? rb.sah / ra : 0.0;
     }
     out.build_ms = std::chrono::duration<double, std::milli>(std::chrono::steady_clock::now() - t0).count();
     return hipSuccess;
@@ -764,14 +1013,54 @@ hipError_t set_transparent_device(Tri3 *tris, uint32_t n, const uint8_t *flags, 
     return hipGetLastError();
 }
 
+hipError_t BvhBuildSpace::reserve(size_t bytes, hipStream_t s)
+{
+    if (bytes <= cap) return hipSuccess;
+    if (dev) {
+        hipError_t e = hipStreamSynchronize(s);
+        if (e != hipSuccess) return e;
+        (void)hipFree(dev);
+        dev = nullptr;
+        cap = 0;
+    }
+    hipError_t e = hipMalloc(&dev, bytes);
+    if (e != hipSuccess) dev = nullptr;
+    else cap = bytes;
+    return e;
+}
+
+hipError_t BvhBuildSpace::reserve_pinned()
+{
+    if (pinned) return hipSuccess;
+    hipError_t e = hipHostMalloc(&pinned, kPinned, hipHostMallocDefault);
+    if (e != hipSuccess) pinned = nullptr;
+    return e;
+}
+
+void BvhBuildSpace::trim(hipStream_t s)
+{
+    if (cap <= kKeep) return;
+    (void)hipStreamSynchronize(s);
+    (void)hipFree(dev);
+    dev = nullptr;
+    cap = 0;
+}
+
+void BvhBuildSpace::release()
+{
+    if (dev) (void)hipFree(dev);
+    if (pinned) (void)hipHostFree(pinned);
+    dev = pinned = nullptr;
+    cap = 0;
+}
+
 void free_bvh_device(DeviceBvhBuild &b)
 {
-    if (b.nodes2) (void)hipFree(b.nodes2);
-    if (b.nodes4) (void)hipFree(b.nodes4);
-    if (b.tris) (void)hipFree(b.tris);
+    if (b.nodes2) (void)hipFree(b.nodes2);  // the whole tree's allocation
     b.nodes2 = nullptr;
     b.nodes4 = nullptr;
     b.tris = nullptr;
+    b.extra = nullptr;
 }
 
 }  // namespace rt

@@ -57,6 +57,42 @@ def test_device_build_equals_oracle(rt, orc, gpu_ctx, n, max_leaf, width, dup):
     bvh.close()
 
 
+def chain(rt, n):
+    """Triangles halving their distance to a corner bit by bit (a radix tree
+    that is a chain down to the last code bit) and n equal ones at its end (equal
+    boxes: the wide nodes open one side only, so the wide tree is about as deep
+    as the two-wide one)."""
+    steps = [0.75 * 2.0**-k * np.eye(3)[a] for k in range(10) for a in range(3)]
+    at = np.concatenate([np.array(steps), np.zeros((n, 3)), np.ones((1, 3))])
+    shape = np.array([[0, 0, 0], [1, 0, 0], [0, 1, 1]]) * 2.0**-13
+    xyz = (at[:, None, :] + shape[None]).astype(np.float32).reshape(-1, 3)
+    return xyz, np.arange(xyz.shape[0], dtype=np.uint32).reshape(-1, 3)
+
+
+@pytest.mark.parametrize("kind,n,max_leaf,width", [
+    # one leaf more and less than one, two and three runs of 512 leaves
+    ("soup", 511, 4, 4), ("soup", 512, 1, 4), ("soup", 513, 4, 4), ("soup", 1025, 8, 2), ("soup", 1537, 4, 4),
+    # more wide levels than are launched before a look (16), at small and large sizes
+    ("chain", 3, 1, 4), ("chain", 513, 1, 4), ("chain", 1 << 17, 1, 4),
+    # a level of more entries than one tile per block (512 x 256)
+    ("soup", 1 << 20, 1, 4)])
+def test_runs_and_levels_equal_the_oracle(rt, orc, gpu_ctx, kind, n, max_leaf, width):
+    print(f"[bvh device] {kind} n={n} max_leaf={max_leaf} width={width}", flush=True)
+    xyz, idx = chain(rt, n) if kind == "chain" else rt.gen_soup(n, seed=n)
+    bvh = device_bvh(rt, gpu_ctx, xyz, idx, max_leaf, width)
+    inf = bvh.info()
+    nodes, tris = bvh.export()
+    want, wn, wt, w4 = orc.lbvh_build(xyz, idx, max_leaf=max_leaf, wide=width == 4)
+    assert (inf.num_nodes, inf.max_depth) == (want["num_nodes"], want["max_depth"])
+    assert np.array_equal(nodes.view(np.uint32), wn.view(np.uint32))
+    assert np.array_equal(tris.view(np.uint32), wt.view(np.uint32))
+    if width == 4:
+        assert (inf.num_nodes4, inf.depth4, inf.stack_cap) == (want["num_nodes4"], want["depth4"],
+                                                               want["max_stack4"] + 1)
+        assert np.array_equal(bvh.export4().view(np.uint32), w4.view(np.uint32))
+    bvh.close()
+
+
 @pytest.mark.parametrize("width", [4, 2])
 @pytest.mark.parametrize("n", [1, 5, 4096, 32768])
 def test_traces_on_device_tree_match_brute_force(rt, orc, gpu_ctx, n, width):
