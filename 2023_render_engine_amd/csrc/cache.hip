@@ -13,10 +13,10 @@
 // sampling/ShapeLightDistribution.cu:20-345).
 //
 // Matmuls run on the matrix cores: v_mfma_f32_16x16x16_bf16 (BF16 inputs,
-// FP32 accumulation).  One wavefront owns a 16-row strip of the output;
-// activations live in HBM between layers as BF16 (64 columns = 128 B per
-// row), weights are read through the L1/L2 caches.  Master weights, Adam
-// moments and gradients are FP32.
+// FP32 accumulation).  One wavefront takes a 16-row strip through all layers
+// in registers, forward (k_infer) and back (k_train_rows); only what the
+// weight gradient reads (k_wgrad) is written to memory, as BF16.  Master
+// weights, Adam moments and gradients are FP32.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -84,148 +84,23 @@ __device__ __forceinline__ void normalise_pos(const CacheDev &c, const float *q,
     pz = fminf(fmaxf((q[2] - c.lo[2]) * c.inv_ext[2], 0.0f), 1.0f);
 }
 
-// X[n][64] (BF16): 2 features per level, normal, view direction, roughness,
-// a constant 1 (the bias-free MLP's offset input) and zero padding.
-__global__ __launch_bounds__(256) void k_encode(CacheDev c, const float *__restrict__ in, uint32_t n,
-                                                const uint32_t *__restrict__ n_dev, uint16_t *__restrict__ X)
-{
-    if (n_dev) n = min(n, *n_dev);
-    for (uint32_t i = blockIdx.x * 256 + threadIdx.x; i < n; i += gridDim.x * 256) {
-        const float *q = in + (size_t)i * kCacheInStride;
-        float px, py, pz;
-        normalise_pos(c, q, px, py, pz);
-        alignas(16) uint16_t row[kCacheWidth];
-        for (uint32_t l = 0; l < c.levels; ++l) {
-            uint32_t idx[8];
-            float w[8];
-            grid_corners(c, l, px, py, pz, idx, w);
-            const uint32_t *tab = (const uint32_t *)c.grid_bf16 + (size_t)l * c.table_size;
-            float f0 = 0, f1 = 0;
-#pragma unroll
-            for (int k = 0; k < 8; ++k) {
-                const uint32_t v = tab[idx[k]];
-                f0 += w[k] * bf2f((uint16_t)(v & 0xffffu));
-                f1 += w[k] * bf2f((uint16_t)(v >> 16));
-            }
-            row[2 * l] = f2bf(f0);
-            row[2 * l + 1] = f2bf(f1);
-        }
-        uint32_t o = 2 * c.levels;
-        for (int k = 3; k < 10; ++k) row[o++] = f2bf(q[k]);  // normal, view dir, roughness
-        row[o++] = f2bf(1.0f);
-        for (; o < kCacheWidth; ++o) row[o] = 0;
-        uint4 *dst = (uint4 *)(X + (size_t)i * kCacheWidth);
-        const uint4 *src = (const uint4 *)row;
-#pragma unroll
-        for (int k = 0; k < kCacheWidth / 8; ++k) dst[k] = src[k];
-    }
-}
+// ---------------------------------------------------------------------
+// weight gradients of all layers: dW[64][NOUT] += X^T dY over all rows, one
+// layer per blockIdx.y.  A workgroup stages 64-row chunks of X and dY in LDS,
+// wave w accumulates dW rows 16w..16w+15 in registers and adds them to the
+// FP32 gradient once at the end.  A staged row takes 72 elements: the 2-byte
+// reads of four rows 4 apart then fall into different banks.
+// ---------------------------------------------------------------------
+constexpr uint32_t kWgradStride = 72;
+// Blocks per layer: 65,536 rows take 8 chunks each.  With 256 or 512 a call
+// took 17 us longer: more chunks at a time, but each block ends in 4096 atomics
+// on the same 16 KB.
+constexpr uint32_t kWgradBlocks = 128;
 
-// ---------------------------------------------------------------------
-// forward layer: Y[n][NOUT] = act(X[n][64] * W), W^T stored [NOUT][64] BF16
-// MODE 0: ReLU, BF16 out (row stride 64); MODE 1: linear, FP32 out (NOUT = 16)
-// ---------------------------------------------------------------------
-template <int NOUT, int MODE>
-__global__ __launch_bounds__(256) void k_fwd(const uint16_t *__restrict__ X, const uint16_t *__restrict__ Wt,
-                                             uint32_t n, const uint32_t *__restrict__ n_dev, void *__restrict__ Y)
-{
-    if (n_dev) n = min(n, *n_dev);
-    const uint32_t lane = __lane_id();
-    const uint32_t wave = threadIdx.x / 64;
-    const uint32_t li = lane & 15, lq = lane >> 4;
-    const uint32_t strips = (n + 15) / 16;
-    for (uint32_t s = blockIdx.x * 4 + wave; s < strips; s += gridDim.x * 4) {
-        const uint32_t row = s * 16 + li;
-        f32x4 acc[NOUT / 16];
-#pragma unroll
-        for (int t = 0; t < NOUT / 16; ++t) acc[t] = f32x4{0, 0, 0, 0};
-#pragma unroll
-        for (int k0 = 0; k0 < kCacheWidth; k0 += 16) {
-            bf16x4 a = {0, 0, 0, 0};
-            if (row < n) a = *(const bf16x4 *)(X + (size_t)row * kCacheWidth + k0 + 4 * lq);
-#pragma unroll
-            for (int t = 0; t < NOUT / 16; ++t) {
-                const bf16x4 b = *(const bf16x4 *)(Wt + (size_t)(t * 16 + li) * kCacheWidth + k0 + 4 * lq);
-                acc[t] = mfma16(a, b, acc[t]);
-            }
-        }
-#pragma unroll
-        for (int t = 0; t < NOUT / 16; ++t)
-#pragma unroll
-            for (int r = 0; r < 4; ++r) {
-                const uint32_t orow = s * 16 + 4 * lq + r;
-                const uint32_t ocol = t * 16 + li;
-                if (orow < n) {
-                    if (MODE == 0)
-                        ((uint16_t *)Y)[(size_t)orow * kCacheWidth + ocol] = f2bf(fmaxf(acc[t][r], 0.0f));
-                    else
-                        ((float *)Y)[(size_t)orow * NOUT + ocol] = acc[t][r];
-                }
-            }
-    }
-}
-
-// ---------------------------------------------------------------------
-// backward through a layer (data gradient):
-//   dX[n][64] = (dY[n][NIN] * W^T) (.) [A > 0]   (A = the layer's input
-//   activation; MASK = 0 for the encoding input, which has no ReLU)
-// W stored [64 in][NIN out] row-major BF16 is the B operand (B[k][j] = W[j][k]).
-// OUTF32 writes FP32 (the encoding gradient), otherwise BF16.
-// ---------------------------------------------------------------------
-template <int NIN, bool MASK, bool OUTF32>
-__global__ __launch_bounds__(256) void k_bwd_data(const uint16_t *__restrict__ dY, const uint16_t *__restrict__ W,
-                                                  const uint16_t *__restrict__ A, uint32_t n,
-                                                  const uint32_t *__restrict__ n_dev, void *__restrict__ dX)
-{
-    if (n_dev) n = min(n, *n_dev);
-    const uint32_t lane = __lane_id();
-    const uint32_t wave = threadIdx.x / 64;
-    const uint32_t li = lane & 15, lq = lane >> 4;
-    const uint32_t strips = (n + 15) / 16;
-    for (uint32_t s = blockIdx.x * 4 + wave; s < strips; s += gridDim.x * 4) {
-        const uint32_t row = s * 16 + li;
-        f32x4 acc[4];
-#pragma unroll
-        for (int t = 0; t < 4; ++t) acc[t] = f32x4{0, 0, 0, 0};
-#pragma unroll
-        for (int k0 = 0; k0 < NIN; k0 += 16) {
-            bf16x4 a = {0, 0, 0, 0};
-            if (row < n) a = *(const bf16x4 *)(dY + (size_t)row * NIN + k0 + 4 * lq);
-#pragma unroll
-            for (int t = 0; t < 4; ++t) {
-                const bf16x4 b = *(const bf16x4 *)(W + (size_t)(t * 16 + li) * NIN + k0 + 4 * lq);
-                acc[t] = mfma16(a, b, acc[t]);
-            }
-        }
-#pragma unroll
-        for (int t = 0; t < 4; ++t)
-#pragma unroll
-            for (int r = 0; r < 4; ++r) {
-                const uint32_t orow = s * 16 + 4 * lq + r;
-                const uint32_t ocol = t * 16 + li;
-                if (orow >= n) continue;
-                float v = acc[t][r];
-                if (MASK && !(bf2f(A[(size_t)orow * kCacheWidth + ocol]) > 0.0f)) v = 0.0f;
-                if (OUTF32)
-                    ((float *)dX)[(size_t)orow * kCacheWidth + ocol] = v;
-                else
-                    ((uint16_t *)dX)[(size_t)orow * kCacheWidth + ocol] = f2bf(v);
-            }
-    }
-}
-
-// ---------------------------------------------------------------------
-// weight gradient: dW[64][NOUT] += X^T dY over all rows.  A workgroup stages
-// 64-row chunks of X and dY in LDS, wave w accumulates dW rows 16w..16w+15
-// in registers and adds them to the FP32 gradient once at the end.
-// ---------------------------------------------------------------------
 template <int NOUT>
-__global__ __launch_bounds__(256) void k_wgrad(const uint16_t *__restrict__ X, const uint16_t *__restrict__ dY,
-                                               uint32_t n, const uint32_t *__restrict__ n_dev, float *__restrict__ dW)
+__device__ __forceinline__ void wgrad_layer(const uint16_t *__restrict__ X, const uint16_t *__restrict__ dY, uint32_t n,
+                                            float *__restrict__ dW, uint16_t *sX, uint16_t *sD)
 {
-    if (n_dev) n = min(n, *n_dev);
-    __shared__ uint16_t sX[64 * kCacheWidth];
-    __shared__ uint16_t sD[64 * NOUT];
     const uint32_t lane = __lane_id();
     const uint32_t wave = threadIdx.x / 64;
     const uint32_t li = lane & 15, lq = lane >> 4;
@@ -240,13 +115,13 @@ __global__ __launch_bounds__(256) void k_wgrad(const uint16_t *__restrict__ X, c
             const uint32_t r = e / (kCacheWidth / 8), c8 = e % (kCacheWidth / 8);
             uint4 v = {0, 0, 0, 0};
             if (r0 + r < n) v = *(const uint4 *)(X + (size_t)(r0 + r) * kCacheWidth + c8 * 8);
-            *(uint4 *)(sX + r * kCacheWidth + c8 * 8) = v;
+            *(uint4 *)(sX + r * kWgradStride + c8 * 8) = v;
         }
         for (uint32_t e = threadIdx.x; e < 64 * NOUT / 8; e += 256) {
             const uint32_t r = e / (NOUT / 8), c8 = e % (NOUT / 8);
             uint4 v = {0, 0, 0, 0};
             if (r0 + r < n) v = *(const uint4 *)(dY + (size_t)(r0 + r) * NOUT + c8 * 8);
-            *(uint4 *)(sD + r * NOUT + c8 * 8) = v;
+            *(uint4 *)(sD + r * kWgradStride + c8 * 8) = v;
         }
         __syncthreads();
         // dW[16w + i][j] += sum_m X[m][16w + i] dY[m][j]; A[i][m] = X[m][16w+i], B[m][j] = dY[m][j]
@@ -254,12 +129,12 @@ __global__ __launch_bounds__(256) void k_wgrad(const uint16_t *__restrict__ X, c
         for (int m0 = 0; m0 < 64; m0 += 16) {
             bf16x4 a;
 #pragma unroll
-            for (int q = 0; q < 4; ++q) a[q] = (short)sX[(m0 + 4 * lq + q) * kCacheWidth + 16 * wave + li];
+            for (int q = 0; q < 4; ++q) a[q] = (short)sX[(m0 + 4 * lq + q) * kWgradStride + 16 * wave + li];
 #pragma unroll
             for (int t = 0; t < NOUT / 16; ++t) {
                 bf16x4 b;
 #pragma unroll
-                for (int q = 0; q < 4; ++q) b[q] = (short)sD[(m0 + 4 * lq + q) * NOUT + t * 16 + li];
+                for (int q = 0; q < 4; ++q) b[q] = (short)sD[(m0 + 4 * lq + q) * kWgradStride + t * 16 + li];
                 acc[t] = mfma16(a, b, acc[t]);
             }
         }
@@ -274,40 +149,15 @@ __global__ __launch_bounds__(256) void k_wgrad(const uint16_t *__restrict__ X, c
         }
 }
 
-// ---------------------------------------------------------------------
-// relative L2 loss (Mueller et al. 2021): l = (y - t)^2 / (sg(y)^2 + 0.01),
-// mean over rows and the 3 channels; writes dY (BF16, [n][16]) and adds the
-// loss sum to *loss.  With n_dev the row count (and the mean's scale) comes
-// from device memory.
-// ---------------------------------------------------------------------
-__global__ __launch_bounds__(256) void k_loss(const float *__restrict__ Y, const float *__restrict__ target,
-                                              uint32_t n, const uint32_t *__restrict__ n_dev, float scale,
-                                              uint16_t *__restrict__ dY, float *__restrict__ loss)
+__global__ __launch_bounds__(256) void k_wgrad(CacheDev c, CacheWork w, uint32_t n, const uint32_t *__restrict__ n_dev)
 {
-    if (n_dev) {
-        n = min(n, *n_dev);
-        scale = n ? 1.0f / (3.0f * (float)n) : 0.0f;
-    }
-    float lsum = 0;
-    for (uint32_t i = blockIdx.x * 256 + threadIdx.x; i < n; i += gridDim.x * 256) {
-        alignas(16) uint16_t g[16];
-#pragma unroll
-        for (int c = 0; c < 16; ++c) g[c] = 0;
-#pragma unroll
-        for (int c = 0; c < 3; ++c) {
-            const float y = Y[(size_t)i * 16 + c], t = target[(size_t)i * 3 + c];
-            const float den = y * y + 0.01f;
-            const float d = y - t;
-            lsum += d * d / den;
-            g[c] = f2bf(2.0f * d / den * scale);
-        }
-        uint4 *dst = (uint4 *)(dY + (size_t)i * 16);
-        dst[0] = ((uint4 *)g)[0];
-        dst[1] = ((uint4 *)g)[1];
-    }
-    // wavefront reduction, one atomic per wavefront
-    for (int off = 32; off > 0; off >>= 1) lsum += __shfl_down(lsum, off);
-    if (__lane_id() == 0 && loss) atomicAdd(loss, lsum);
+    __shared__ uint16_t sX[64 * kWgradStride], sD[64 * kWgradStride];
+    if (n_dev) n = min(n, *n_dev);
+    const uint32_t l = blockIdx.y;
+    if (l + 1 < kCacheLayers)
+        wgrad_layer<kCacheWidth>(w.act[l], w.dact[l], n, c.grad + kCacheLayerOffset(l), sX, sD);
+    else
+        wgrad_layer<kCacheOut>(w.act[l], w.dy16, n, c.grad + kCacheLayerOffset(l), sX, sD);
 }
 
 // Morton key of each sample's normalised position (10 bits per axis; rows
@@ -338,68 +188,71 @@ __global__ __launch_bounds__(256) void k_sample_morton(CacheDev c, const float *
     }
 }
 
-// hash-grid gradient: scatter dX[:, 0..2L) through the trilinear weights.
-// Block (level l, run jb) takes the samples at positions jb*256 .. +255 of
-// the batch's Morton order, so its lanes sit close together in space and
-// share grid cells on all but the finest levels.  Their 8 corner updates
-// are first merged in an LDS table keyed by cell (open addressing, 4096
-// slots for at most 2048 distinct cells, so a probe always ends), and each
-// distinct cell then takes one device-scope atomic per feature: on a
-// surface-sampled batch that is 2.4x fewer atomics overall and 50-130x fewer
-// on the coarse levels, where one atomic per corner serialised on a few
-// thousand addresses.
-constexpr uint32_t kGridSlots = 4096;
+// hash-grid gradient: scatter the features' gradients through the trilinear
+// weights.  Block (level l, run jb) takes the samples at positions jb*256 ..
+// +255 of the batch's Morton order, so its lanes sit close together in space
+// and share grid cells on all but the finest levels.  Their 8 corner updates
+// are first merged in an LDS table keyed by pairs of cells 2k, 2k + 1 (open
+// addressing, 2048 slots for at most 2048 distinct pairs, so a probe always
+// ends): on a surface-sampled batch that is 2.4x fewer atomics overall and
+// 50-130x fewer on the coarse levels, where one atomic per corner serialised
+// on a few thousand addresses.
+//
+// What bounds it: the requests of the device-scope atomics.  A pair's four
+// sums are added by four neighbouring lanes, whose words lie in one cache
+// line, so they are one request; corners one x apart are mostly a pair (in a
+// hashed level where x is even).  65,536 uniform samples, 16 levels of 2^15
+// entries: 194 us, against 387 us keyed by single cells, one lane adding a
+// cell's two features in turn and the gradients read from rows of 256 B.
+constexpr uint32_t kGridPairs = 2048;
 constexpr uint32_t kGridEmpty = 0xffffffffu;
 
 __global__ __launch_bounds__(256) void k_grid_bwd(CacheDev c, const float *__restrict__ in, uint32_t n,
                                                   const uint32_t *__restrict__ n_dev, uint32_t runs,
-                                                  const uint32_t *__restrict__ order, const float *__restrict__ dX,
-                                                  float *__restrict__ dgrid)
+                                                  const uint32_t *__restrict__ order, const float2 *__restrict__ dfeat,
+                                                  uint32_t rows, float *__restrict__ dgrid)
 {
-    __shared__ uint32_t skey[kGridSlots];
-    __shared__ float sv0[kGridSlots], sv1[kGridSlots];
+    __shared__ uint32_t skey[kGridPairs];
+    __shared__ float sv[kGridPairs * 4];
     const uint32_t count = n_dev ? min(n, *n_dev) : n;
     const uint32_t l = blockIdx.x / runs, jb = blockIdx.x - l * runs;
     if (l >= c.levels || jb * 256 >= count) return;  // whole block: before any barrier
-    for (uint32_t t = threadIdx.x; t < kGridSlots; t += 256) {
-        skey[t] = kGridEmpty;
-        sv0[t] = 0.0f;
-        sv1[t] = 0.0f;
-    }
+    for (uint32_t t = threadIdx.x; t < kGridPairs; t += 256) skey[t] = kGridEmpty;
+    for (uint32_t t = threadIdx.x; t < kGridPairs; t += 256) ((float4 *)sv)[t] = make_float4(0, 0, 0, 0);
     __syncthreads();
     const uint32_t j = jb * 256 + threadIdx.x;
     if (j < count) {
         const uint32_t i = order[j];
-        const float g0 = dX[(size_t)i * kCacheWidth + 2 * l], g1 = dX[(size_t)i * kCacheWidth + 2 * l + 1];
-        if (g0 != 0.0f || g1 != 0.0f) {
+        const float2 g = dfeat[(size_t)l * rows + i];
+        if (g.x != 0.0f || g.y != 0.0f) {
             float px, py, pz;
             normalise_pos(c, in + (size_t)i * kCacheInStride, px, py, pz);
             uint32_t idx[8];
             float w[8];
             grid_corners(c, l, px, py, pz, idx, w);
+            uint32_t h = 0;
 #pragma unroll
             for (int k = 0; k < 8; ++k) {
-                uint32_t h = (idx[k] * 2654435761u) >> 20;  // 12 bits
-                for (;;) {
-                    const uint32_t prev = atomicCAS(&skey[h], kGridEmpty, idx[k]);
-                    if (prev == kGridEmpty || prev == idx[k]) {
-                        atomicAdd(&sv0[h], w[k] * g0);
-                        atomicAdd(&sv1[h], w[k] * g1);
-                        break;
+                const uint32_t pair = idx[k] >> 1;
+                if (!(k & 1) || pair != idx[k - 1] >> 1) {
+                    h = (pair * 2654435761u) >> 21;  // 11 bits
+                    for (;;) {
+                        const uint32_t prev = atomicCAS(&skey[h], kGridEmpty, pair);
+                        if (prev == kGridEmpty || prev == pair) break;
+                        h = (h + 1) & (kGridPairs - 1);
                     }
-                    h = (h + 1) & (kGridSlots - 1);
                 }
+                float *v = sv + 4 * h + 2 * (idx[k] & 1u);
+                atomicAdd(v, w[k] * g.x);
+                atomicAdd(v + 1, w[k] * g.y);
             }
         }
     }
     __syncthreads();
     float *tab = dgrid + (size_t)l * c.table_size * 2;
-    for (uint32_t t = threadIdx.x; t < kGridSlots; t += 256) {
-        const uint32_t key = skey[t];
-        if (key != kGridEmpty) {
-            atomicAdd(&tab[2 * (size_t)key], sv0[t]);
-            atomicAdd(&tab[2 * (size_t)key + 1], sv1[t]);
-        }
+    for (uint32_t t = threadIdx.x; t < kGridPairs * 4; t += 256) {
+        const float v = sv[t];
+        if (v != 0.0f) atomicAdd(&tab[4 * (size_t)skey[t >> 2] + (t & 3u)], v);
     }
 }
 
@@ -649,6 +502,134 @@ __global__ __launch_bounds__(256) void k_infer(CacheDev c, const float *__restri
 }
 
 // ---------------------------------------------------------------------
+// Training: encoding, forward, loss and data gradients of a 16-row strip in
+// one wavefront, in k_infer's layout.  The backward products are transposed the
+// same way, dX^T = W dY^T, with W (in x out) as the A operand.  The loss is the
+// relative L2 loss of Mueller et al. 2021: l = (y - t)^2 / (sg(y)^2 + 0.01),
+// mean over rows and the 3 channels (with n_dev the count, and so the mean's
+// scale, comes from device memory).  What the weight gradient needs goes to
+// memory as BF16: every layer's input act[l] and its masked output gradient
+// dact[l] (dy16 for the output layer); the encoding's gradient as FP32, one
+// float2 per level and row.
+//
+// Both weight layouts (70 KB) stay in LDS: a wavefront has one or two strips
+// of a batch, so registers would only be filled once or twice.  65,536 rows:
+// 74 us (bound by its chain of gathers, products and stores at two wavefronts
+// per SIMD), against 159 us in twelve kernels; with k_wgrad 100 us against 247.
+// ---------------------------------------------------------------------
+__device__ __forceinline__ void load_backward_frags(const CacheDev &c, uint2 *frags)
+{
+    for (uint32_t e = threadIdx.x; e < kCacheFrags * 64; e += blockDim.x) {
+        const uint32_t f = e >> 6, l = e & 63u;
+        const uint32_t layer = f >> 4, o = f < 64 ? (f >> 2) & 3u : f & 3u, k = f < 64 ? f & 3u : 0u;
+        const uint32_t nout = f < 64 ? kCacheWidth : kCacheOut;
+        frags[e] = *(const uint2 *)(c.w + kCacheLayerOffset(layer) + (16 * o + (l & 15u)) * nout + 16 * k + 4 * (l >> 4));
+    }
+}
+
+__device__ __forceinline__ bf16x4 pack4(const f32x4 &v)
+{
+    return __builtin_bit_cast(bf16x4, make_uint2(pack_bf16(v[0], v[1]), pack_bf16(v[2], v[3])));
+}
+
+// v where the activation a is positive, else 0.
+__device__ __forceinline__ f32x4 relu_mask(f32x4 v, bf16x4 a)
+{
+#pragma unroll
+    for (int r = 0; r < 4; ++r)
+        if (!(bf2f((uint16_t)a[r]) > 0.0f)) v[r] = 0.0f;
+    return v;
+}
+
+__device__ __forceinline__ void store_strip(uint16_t *dst, uint32_t row, uint32_t q, const bf16x4 x[4])
+{
+#pragma unroll
+    for (int t = 0; t < 4; ++t) *(bf16x4 *)(dst + (size_t)row * kCacheWidth + 16 * t + 4 * q) = x[t];
+}
+
+__global__ __launch_bounds__(256) void k_train_rows(CacheDev c, CacheWork w, const float *__restrict__ in,
+                                                    const float *__restrict__ target, uint32_t n,
+                                                    const uint32_t *__restrict__ n_dev, float scale,
+                                                    float *__restrict__ loss)
+{
+    __shared__ uint2 fw[kCacheFrags * 64], bw[kCacheFrags * 64];
+    if (n_dev) {
+        n = min(n, *n_dev);
+        scale = n ? 1.0f / (3.0f * (float)n) : 0.0f;
+    }
+    const uint32_t strips = (n + 15) / 16;
+    if (blockIdx.x * 4 >= strips) return;  // whole block: before the barrier
+    load_weight_frags(c, fw);
+    load_backward_frags(c, bw);
+    __syncthreads();
+    const uint32_t lane = __lane_id(), wave = threadIdx.x / 64, q = lane >> 4;
+    const LaneLevels ll = lane_levels(c, q);
+    float lsum = 0;
+    for (uint32_t s = blockIdx.x * 4 + wave; s < strips; s += gridDim.x * 4) {
+        uint32_t at = lane;
+        asm volatile("" : "+v"(at));  // the fragments are read for every strip
+        const uint32_t row = s * 16 + (lane & 15u);
+        const bool valid = row < n;
+        bf16x4 a[kCacheLayers][4];
+        encode_strip(c, ll, in + (size_t)min(row, n - 1) * kCacheInStride, q, a[0]);
+        if (valid) store_strip(w.act[0], row, q, a[0]);
+#pragma unroll
+        for (uint32_t l = 0; l + 1 < kCacheLayers; ++l) {
+#pragma unroll
+            for (int t = 0; t < 4; ++t) a[l + 1][t] = a[l][t];
+            hidden_layer(fw, l, at, a[l + 1]);
+            if (valid) store_strip(w.act[l + 1], row, q, a[l + 1]);
+        }
+        const f32x4 y = output_layer(fw, at, a[kCacheLayers - 1]);
+        f32x4 g{0, 0, 0, 0};
+        if (q == 0 && valid) {
+#pragma unroll
+            for (int k = 0; k < 3; ++k) {
+                const float t = target[(size_t)row * 3 + k];
+                const float den = y[k] * y[k] + 0.01f;
+                const float d = y[k] - t;
+                lsum += d * d / den;
+                g[k] = 2.0f * d / den * scale;
+            }
+        }
+        const bf16x4 dy = pack4(g);
+        if (valid) *(bf16x4 *)(w.dy16 + (size_t)row * kCacheOut + 4 * q) = dy;
+        bf16x4 d[4];
+#pragma unroll
+        for (int o = 0; o < 4; ++o)
+            d[o] = pack4(relu_mask(mfma16(__builtin_bit_cast(bf16x4, bw[(64 + o) * 64 + at]), dy, f32x4{0, 0, 0, 0}),
+                                   a[kCacheLayers - 1][o]));
+#pragma unroll
+        for (int l = (int)kCacheLayers - 2; l >= 0; --l) {
+            if (valid) store_strip(w.dact[l], row, q, d);
+            f32x4 acc[4];
+#pragma unroll
+            for (int o = 0; o < (l ? 4 : 2); ++o) {
+                acc[o] = f32x4{0, 0, 0, 0};
+#pragma unroll
+                for (int k = 0; k < 4; ++k)
+                    acc[o] = mfma16(__builtin_bit_cast(bf16x4, bw[(l * 16 + o * 4 + k) * 64 + at]), d[k], acc[o]);
+            }
+            if (l) {
+#pragma unroll
+                for (int o = 0; o < 4; ++o) d[o] = pack4(relu_mask(acc[o], a[l][o]));
+            } else if (valid) {
+                // features 16o + 4q + 0..3 are levels 8o + 2q and the next
+#pragma unroll
+                for (uint32_t i = 0; i < 4; ++i) {
+                    const uint32_t lev = 8 * (i >> 1) + 2 * q + (i & 1u);
+                    if (lev < c.levels)
+                        w.dfeat[(size_t)lev * w.rows + row] = make_float2(acc[i >> 1][2 * (i & 1u)], acc[i >> 1][2 * (i & 1u) + 1]);
+                }
+            }
+        }
+    }
+    // wavefront reduction, one atomic per wavefront
+    for (int off = 32; off > 0; off >>= 1) lsum += __shfl_down(lsum, off);
+    if (lane == 0 && loss) atomicAdd(loss, lsum);
+}
+
+// ---------------------------------------------------------------------
 // host launchers
 // ---------------------------------------------------------------------
 static dim3 grid_for(uint32_t work, uint32_t per_block, uint32_t cap = 4096)
@@ -657,21 +638,6 @@ static dim3 grid_for(uint32_t work, uint32_t per_block, uint32_t cap = 4096)
     if (b < 1) b = 1;
     if (b > cap) b = cap;
     return dim3(b);
-}
-
-hipError_t cache_forward(const CacheDev &c, const CacheWork &w, const float *in, uint32_t n, hipStream_t s,
-                         const uint32_t *n_dev)
-{
-    if (n == 0) return hipSuccess;
-    const dim3 blk(256);
-    hipLaunchKernelGGL(k_encode, grid_for(n, 256), blk, 0, s, c, in, n, n_dev, w.act[0]);
-    const dim3 g = grid_for((n + 15) / 16, 4);
-    for (uint32_t l = 0; l + 1 < kCacheLayers; ++l)
-        hipLaunchKernelGGL((k_fwd<64, 0>), g, blk, 0, s, w.act[l], c.w_t + kCacheLayerOffset(l), n, n_dev,
-                           (void *)w.act[l + 1]);
-    hipLaunchKernelGGL((k_fwd<16, 1>), g, blk, 0, s, w.act[kCacheLayers - 1],
-                       c.w_t + kCacheLayerOffset(kCacheLayers - 1), n, n_dev, (void *)w.y);
-    return hipGetLastError();
 }
 
 hipError_t cache_infer(const CacheDev &c, const float *in, uint32_t n, float *rgb, hipStream_t s,
@@ -692,39 +658,19 @@ hipError_t cache_backward(const CacheDev &c, const CacheWork &w, const float *in
 {
     if (n == 0) return hipSuccess;
     const dim3 blk(256);
-    hipError_t e = cache_forward(c, w, in, n, s, n_dev);
-    if (e != hipSuccess) return e;
-    hipLaunchKernelGGL(k_loss, grid_for(n, 256), blk, 0, s, w.y, target, n, n_dev, 1.0f / (3.0f * (float)n), w.dy16,
-                       loss);
-    const dim3 g = grid_for((n + 15) / 16, 4);
-    const dim3 gw = grid_for((n + 63) / 64, 1, 512);
-    const uint32_t L = kCacheLayers;
-    // output layer
-    hipLaunchKernelGGL((k_wgrad<16>), gw, blk, 0, s, w.act[L - 1], w.dy16, n, n_dev, c.grad + kCacheLayerOffset(L - 1));
-    hipLaunchKernelGGL((k_bwd_data<16, true, false>), g, blk, 0, s, w.dy16, c.w + kCacheLayerOffset(L - 1),
-                       w.act[L - 1], n, n_dev, (void *)w.dact[0]);
-    // hidden layers l = L-2 .. 1: input act[l], output grad in dact
-    uint32_t cur = 0;
-    for (int l = (int)L - 2; l >= 1; --l) {
-        hipLaunchKernelGGL((k_wgrad<64>), gw, blk, 0, s, w.act[l], w.dact[cur], n, n_dev,
-                           c.grad + kCacheLayerOffset(l));
-        hipLaunchKernelGGL((k_bwd_data<64, true, false>), g, blk, 0, s, w.dact[cur], c.w + kCacheLayerOffset(l),
-                           w.act[l], n, n_dev, (void *)w.dact[cur ^ 1]);
-        cur ^= 1;
-    }
-    // first layer: weight gradient and the encoding gradient (FP32)
-    hipLaunchKernelGGL((k_wgrad<64>), gw, blk, 0, s, w.act[0], w.dact[cur], n, n_dev, c.grad + kCacheLayerOffset(0));
-    hipLaunchKernelGGL((k_bwd_data<64, false, true>), g, blk, 0, s, w.dact[cur], c.w + kCacheLayerOffset(0),
-                       w.act[0], n, n_dev, (void *)w.dx32);
+    // four strips of 16 rows per block and turn, two blocks per CU
+    hipLaunchKernelGGL(k_train_rows, grid_for((n + 15) / 16, 4, 512), blk, 0, s, c, w, in, target, n, n_dev,
+                       1.0f / (3.0f * (float)n), loss);
+    hipLaunchKernelGGL(k_wgrad, dim3(grid_for((n + 63) / 64, 1, kWgradBlocks).x, kCacheLayers), blk, 0, s, c, w, n, n_dev);
     // the grid gradient in Morton order of the samples' positions
     hipLaunchKernelGGL(k_sample_morton, grid_for(n, 256), blk, 0, s, c, in, n, n_dev, w.skey[0], w.sidx[0]);
     size_t tb = w.sort_bytes;
-    e = hipcub::DeviceRadixSort::SortPairs(w.sort_tmp, tb, w.skey[0], w.skey[1], w.sidx[0], w.sidx[1], (int)n, 0, 32,
+    hipError_t e = hipcub::DeviceRadixSort::SortPairs(w.sort_tmp, tb, w.skey[0], w.skey[1], w.sidx[0], w.sidx[1], (int)n, 0, 32,
                                            s);
     if (e != hipSuccess) return e;
     const uint32_t runs = (n + 255) / 256;
-    hipLaunchKernelGGL(k_grid_bwd, dim3(runs * c.levels), blk, 0, s, c, in, n, n_dev, runs, w.sidx[1], w.dx32,
-                       c.grid_grad);
+    hipLaunchKernelGGL(k_grid_bwd, dim3(runs * c.levels), blk, 0, s, c, in, n, n_dev, runs, w.sidx[1], w.dfeat,
+                       w.rows, c.grid_grad);
     return hipGetLastError();
 }
 

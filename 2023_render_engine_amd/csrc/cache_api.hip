@@ -174,9 +174,10 @@ rt_status rt_cache_create(rt_ctx *ctx, const rt_cache_opts *opts, rt_cache **out
                  o_gv = take(gp * 4);
     size_t o_act[rt::kCacheLayers];
     for (uint32_t l = 0; l < rt::kCacheLayers; ++l) o_act[l] = take((size_t)rows * rt::kCacheWidth * 2);
-    const size_t o_y = take((size_t)rows * 16 * 4), o_dy = take((size_t)rows * 16 * 2);
-    const size_t o_da0 = take((size_t)rows * 64 * 2), o_da1 = take((size_t)rows * 64 * 2);
-    const size_t o_dx = take((size_t)rows * 64 * 4), o_loss = take(4);
+    const size_t o_dy = take((size_t)rows * rt::kCacheOut * 2);
+    size_t o_da[rt::kCacheLayers - 1];
+    for (size_t &o_d : o_da) o_d = take((size_t)rows * rt::kCacheWidth * 2);
+    const size_t o_df = take((size_t)rows * d.levels * 8), o_loss = take(4);
     const size_t sort_bytes = std::max<size_t>(rt::cache_sort_bytes(rows), 1);
     const size_t o_sk0 = take((size_t)rows * 4), o_sk1 = take((size_t)rows * 4), o_si0 = take((size_t)rows * 4),
                  o_si1 = take((size_t)rows * 4), o_stmp = take(sort_bytes);
@@ -196,11 +197,9 @@ rt_status rt_cache_create(rt_ctx *ctx, const rt_cache_opts *opts, rt_cache **out
     rt::CacheWork &w = c->work;
     w.rows = rows;
     for (uint32_t l = 0; l < rt::kCacheLayers; ++l) w.act[l] = (uint16_t *)(base + o_act[l]);
-    w.y = (float *)(base + o_y);
     w.dy16 = (uint16_t *)(base + o_dy);
-    w.dact[0] = (uint16_t *)(base + o_da0);
-    w.dact[1] = (uint16_t *)(base + o_da1);
-    w.dx32 = (float *)(base + o_dx);
+    for (uint32_t l = 0; l + 1 < rt::kCacheLayers; ++l) w.dact[l] = (uint16_t *)(base + o_da[l]);
+    w.dfeat = (float2 *)(base + o_df);
     w.skey[0] = (uint32_t *)(base + o_sk0);
     w.skey[1] = (uint32_t *)(base + o_sk1);
     w.sidx[0] = (uint32_t *)(base + o_si0);

@@ -39,10 +39,9 @@ struct CacheOptsDev {
 struct CacheWork {
     uint32_t rows;
     uint16_t *act[kCacheLayers];  // act[0] = encoding, act[l] = ReLU output of layer l-1
-    float *y;                     // [rows][16] output layer
     uint16_t *dy16;               // [rows][16] loss gradient
-    uint16_t *dact[2];            // [rows][64] ping-pong data gradients
-    float *dx32;                  // [rows][64] encoding gradient
+    uint16_t *dact[kCacheLayers - 1];  // dact[l]: [rows][64] gradient at layer l's output, before its ReLU
+    float2 *dfeat;                // [levels][rows] gradient of the encoding's grid features
     // the grid gradient visits the batch in Morton order of position:
     // keys and sample indices (two buffers each for the sort) and the sort's
     // temporary storage (cache_sort_bytes(rows) bytes)
@@ -57,8 +56,6 @@ size_t cache_sort_bytes(uint32_t rows);
 // n is the row count (and grid size); with n_dev the kernels read the
 // actual count from device memory (capped at n), so a launch sequence can be
 // fixed before the count is known.
-hipError_t cache_forward(const CacheDev &c, const CacheWork &w, const float *in, uint32_t n, hipStream_t s,
-                         const uint32_t *n_dev = nullptr);
 // rgb = max(MLP(encoding(in)), 0) for any n; needs no scratch.
 hipError_t cache_infer(const CacheDev &c, const float *in, uint32_t n, float *rgb, hipStream_t s,
                        const uint32_t *n_dev = nullptr);

@@ -134,3 +134,30 @@ def test_query_sizes_and_level_counts(rt, gpu_ctx, orc, levels, log2_table, base
     ref = np.maximum(ref, 0)
     assert np.max(np.abs(y[at] - ref)) <= 1e-2 * max(1.0, np.max(np.abs(ref)))
     cache.close()
+
+
+@pytest.mark.parametrize("levels,log2_table,base,scale", [(1, 8, 2, 1.0), (3, 9, 7, 1.7), (5, 12, 4, 2.0), (16, 15, 16, 1.38)])
+@pytest.mark.parametrize("n", [1, 15, 17, 64, 65, 257, 1000])
+def test_gradient_sizes_and_level_counts(rt, gpu_ctx, orc, levels, log2_table, base, scale, n):
+    """Strips of 16 rows, chunks of 64 and runs of 256 with remainders, level
+    counts that end inside a feature tile, nearly as many distinct cells in a run
+    as its merge table holds (16 levels), positions on the box's faces (both
+    corners of a pair in one cell).  Five BF16 storage points in series, each
+    off by at most one rounding (2^-8) from the oracle's: 5 * 2^-8 < 2e-2."""
+    cache = rt.RadianceCache(gpu_ctx, (0, 0, 0), (1, 1, 1), levels=levels, log2_table=log2_table, base_res=base,
+                             per_level_scale=scale, batch=1000, seed=3)
+    cfg = orc.cache_cfg(levels, log2_table, base, scale, (0, 0, 0), (1, 1, 1))
+    mlp, grid = cache.get_params()
+    grid = np.random.default_rng(11).uniform(-0.5, 0.5, grid.shape).astype(np.float32)
+    cache.set_params(mlp, grid)
+    rec = records(n, 5)
+    rec[:: 7, 0] = 1.0
+    rec[3:: 7, 1] = 0.0
+    rec[5:: 7, 2] = 1.0
+    tgt = np.random.default_rng(6).uniform(0, 2, (n, 3)).astype(np.float32)
+    loss, mg, gg = cache.gradients(torch.from_numpy(rec).cuda(), torch.from_numpy(tgt).cuda())
+    l_ref, mg_ref, gg_ref, _ = orc.cache_loss_grad(cfg, mlp, grid, rec, tgt, emulate_bf16=True)
+    assert abs(loss - l_ref) <= 1e-2 * l_ref
+    assert rel_err(mg, mg_ref) < 2e-2
+    assert rel_err(gg, gg_ref) < 2e-2
+    cache.close()
