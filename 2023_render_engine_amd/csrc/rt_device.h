@@ -183,20 +183,10 @@ __device__ __forceinline__ void decode_leaf(int32_t c, uint32_t &first, uint32_t
 // which bounds the pending entries, so it cannot overflow.
 // ---------------------------------------------------------------------
 constexpr int kTravBlock = 128;
-// Tuning constants of the persistent traversal (build-time, -D overridable).
-#ifndef RT_REFILL_LANES
-#define RT_REFILL_LANES 16
-#endif
-#ifndef RT_CLAIM_CHUNK
-#define RT_CLAIM_CHUNK 128
-#endif
-#ifndef RT_CLAIM_MIN
-#define RT_CLAIM_MIN 64
-#endif
+// Tuning constant of the persistent traversal (build-time, -D overridable).
 #ifndef RT_NODE_STEPS
 #define RT_NODE_STEPS 4
 #endif
-constexpr uint32_t kRefillLanes = RT_REFILL_LANES;  // refill a wavefront when at least this many lanes are idle
 
 // The traversal stack of a lane: its first L entries in LDS ([depth][lane],
 // stride kTravBlock), deeper ones (up to kMaxStack, the most pending entries
@@ -557,7 +547,7 @@ __device__ __forceinline__ bool trav_step_any(TravState &s, const float4 *__rest
 // on one XCD and its L2), and a persistent wavefront that finds its stripe
 // drained claims work from the others.
 // ---------------------------------------------------------------------
-// kStripes and kCtrStride are in rt_trace.h (the host sizes the counters)
+// kStripes and kCtrStride are in rt_deal.h (the host sizes the counters)
 static_assert(kStripes == 64, "stripe scans use one wavefront lane per stripe");
 
 // A persistent wavefront's position in the stripes (wavefront-uniform).
@@ -569,9 +559,6 @@ static_assert(kStripes == 64, "stripe scans use one wavefront lane per stripe");
 // of queueing two or more rays on each lane of a few wavefronts.  The
 // wavefront hands claimed items to its idle lanes from the local range
 // [lb, le) of stripe ls, so partial refills cost no atomic.
-constexpr uint32_t kClaimChunk = RT_CLAIM_CHUNK;
-constexpr uint32_t kClaimMin = RT_CLAIM_MIN;
-static_assert(kClaimMin >= 1 && kClaimMin <= kClaimChunk, "claim sizes run from kClaimMin to kClaimChunk");
 
 struct StripeCursor {
     uint32_t s;       // stripe being claimed from
@@ -589,13 +576,6 @@ struct StripeCursor {
 // is handed out.
 __device__ __forceinline__ bool cursor_finished(const StripeCursor &c) { return c.done && c.lb == c.le; }
 
-// A launch with fewer items than kWidthWaves full wavefronts (two per SIMD)
-// takes them with fewer lanes of more wavefronts, down to kMinWidth: a small
-// launch is as long as its slowest wavefront, and a wavefront runs through the
-// node and leaf work of all its rays in turn.  8192 rays against 4096
-// triangles, closest and any hit: 248 us with 64 lanes, 224 with 16, 214 with
-// 4; cached 960x540 frames 7.28 and 7.03 ms with 64 and 4.
-constexpr uint32_t kWidthWaves = 2048, kMinWidth = 4;
 template <class Count>
 __device__ __forceinline__ void cursor_init(StripeCursor &c, uint32_t home, Count count)
 {
@@ -603,9 +583,7 @@ __device__ __forceinline__ void cursor_init(StripeCursor &c, uint32_t home, Coun
     uint32_t total = mine;
 #pragma unroll
     for (int off = 32; off > 0; off >>= 1) total += (uint32_t)__shfl_xor((int)total, off);
-    const uint32_t waves = min(gridDim.x * (blockDim.x >> 6), kWidthWaves);
-    c.width = 64u;
-    while (c.width > kMinWidth && total <= (c.width >> 1) * waves) c.width >>= 1;
+    c.width = deal_width(total, gridDim.x * (blockDim.x >> 6));
     c.s = home;
     c.n = (uint32_t)__shfl((int)mine, (int)home);
     c.left = c.n;
@@ -616,9 +594,8 @@ __device__ __forceinline__ void cursor_init(StripeCursor &c, uint32_t home, Coun
     c.lb = 0;
     c.le = 0;
     c.empty = c.n == 0;
-    // in a small launch a stripe's own wavefronts suffice: the rest leave
     const uint32_t nth = (blockIdx.x / kStripes) * (blockDim.x >> 6) + (threadIdx.x >> 6);
-    c.done = total == 0 || (c.width < 64u && nth * c.width >= c.n);
+    c.done = total == 0 || deal_leaves(c.width, nth, c.n);
 }
 
 // Lanes at a parked leaf that start a leaf phase: a quarter of those that take items.
@@ -664,12 +641,11 @@ __device__ __forceinline__ bool cursor_scan(StripeCursor &c, uint32_t *fetch, Co
 // Items of the next claim (wavefront-uniform).
 __device__ __forceinline__ uint32_t claim_size(const StripeCursor &c)
 {
-    const uint32_t k = c.left >> c.wlog, least = min(kClaimMin, c.width);
-    return k < least ? least : (k > kClaimChunk ? kClaimChunk : k);
+    return deal_claim(c.left, c.wlog, c.width);
 }
 
-// Wavefront-uniform refill of idle lanes: when at least kRefillLanes lanes
-// are idle (or all are), they take consecutive items of the local range;
+// Wavefront-uniform refill of idle lanes: when at least deal_refill of the
+// lanes that take items are idle, they take consecutive items of the local range;
 // an empty local range is first refilled with one atomic claim of
 // claim_size items from the cursor's stripe.  Returns the lane's item
 // offset within `stripe`, or UINT32_MAX.  The claim loop is
@@ -682,7 +658,7 @@ __device__ __forceinline__ uint32_t wave_claim(StripeCursor &c, uint32_t *fetch,
     const uint32_t lane = __lane_id();
     const uint64_t idle = __ballot(!has && lane < c.width);
     const uint32_t nidle = (uint32_t)__popcll(idle);
-    if (nidle < (c.width * kRefillLanes) >> 6) return 0xffffffffu;
+    if (nidle < deal_refill(c.width)) return 0xffffffffu;
     if (c.lb == c.le) {
         if (c.done) return 0xffffffffu;
         const uint32_t leader = (uint32_t)(__ffsll((unsigned long long)idle) - 1);

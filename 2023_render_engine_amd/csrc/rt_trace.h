@@ -4,14 +4,10 @@
 #include <hip/hip_runtime.h>
 #include <cstdint>
 
+#include "rt_deal.h"
+
 namespace rt {
 
-// Work striping of the persistent kernels and the wavefront queues: work is
-// cut into kStripes stripes whose counters sit kCtrStride u32 words (one
-// 128-byte line) apart, so device atomics spread over 64 addresses.
-constexpr uint32_t kStripes = 64;
-constexpr uint32_t kCtrStride = 32;
-constexpr uint32_t kClaimWords = kStripes * kCtrStride;  // one striped counter set
 // Largest traversal-stack bound (pending entries per lane) the kernels hold:
 // the first entries in LDS, the rest in the lane's private memory.
 constexpr uint32_t kMaxTraversalStack = 128;

@@ -24,6 +24,7 @@
 namespace rt {
 
 constexpr int kTraceBlock = kTravBlock;
+static_assert(kTraceBlock == 64 * kWavesPerBlock, "ray_deal counts the wavefronts of a workgroup");
 
 __device__ __forceinline__ void trav_init(TravState &s, const RaysDev &rays, uint32_t i, bool any)
 {
@@ -49,19 +50,7 @@ __global__ __launch_bounds__(kTraceBlock) void k_trace(const float4 *__restrict_
     StackTail<TraceStack> s_tail;
     const TraceStack stack{s_stack + threadIdx.x, s_tail};
     stack_init(stack);
-    // the rays are dealt to the stripes in chunks of 2^lc consecutive rays
-    // (chunk c to stripe c % kStripes), so every stripe holds a sample of
-    // the whole batch and the stripes take about equally long
-    const uint32_t nfull = n >> lc, rem = n & ((1u << lc) - 1u);
-    const uint32_t last = nfull & (kStripes - 1u);
-    auto count = [&](uint32_t j) {
-        uint32_t k = ((nfull >> 6) + (j < last ? 1u : 0u)) << lc;
-        if (rem && j == last) k += rem;
-        return k;
-    };
-    auto ray_of = [&](uint32_t j, uint32_t off) {
-        return ((((off >> lc) << 6) + j) << lc) + (off & ((1u << lc) - 1u));
-    };
+    auto count = [&](uint32_t j) { return deal_count(n, lc, j); };
     StripeCursor cur;
     cursor_init(cur, blockIdx.x % kStripes, count);
     TravState s;
@@ -72,7 +61,7 @@ __global__ __launch_bounds__(kTraceBlock) void k_trace(const float4 *__restrict_
         uint32_t stripe = 0;
         const uint32_t r = wave_claim(cur, ray_counter, count, has, stripe);
         if (r != 0xffffffffu) {
-            ray = ray_of(stripe, r);
+            ray = deal_ray(lc, stripe, r);
             trav_init(s, rays, ray, ANY);
             has = true;
         }
@@ -110,23 +99,18 @@ hipError_t launch_trace(const DevBvh &bvh, const RaysDev &rays, uint32_t n, int3
         if (e != hipSuccess || g_cus <= 0) g_cus = 256;
     }
     const int cap = (int)bvh.stack_cap;
-    // stripe chunk 2^lc: a power of two in [64, 4096], about n / 2048 rays
-    uint32_t lc = 6;
-    while (lc < 12 && ((uint64_t)2048 << lc) <= n) ++lc;
     const size_t lds = trace_lds_bytes(bvh.stack_cap);
     // persistent launch: as many workgroups as fit (LDS-limited, at most 16
     // per CU), never more than the rays need
     size_t per_cu = lds ? (160u * 1024u) / lds : 16;
     if (per_cu > 16) per_cu = 16;
     if (per_cu < 1) per_cu = 1;
-    size_t blocks = (size_t)g_cus * per_cu;
-    const size_t need = ((size_t)n + 2 * kMinWidth - 1) / (2 * kMinWidth);
-    if (blocks > need) blocks = need;
-    const dim3 grid((unsigned)blocks);
+    const RayDeal deal = ray_deal(n, (uint32_t)(g_cus * per_cu));
+    const dim3 grid(deal.blocks);
     const float4 *nd = (const float4 *)bvh.nodes, *tr = (const float4 *)bvh.tris;
     auto go = [&](auto kern) {
         hipLaunchKernelGGL(kern, grid, dim3(kTraceBlock), lds, stream, nd, tr, rays, n, prim, t, occluded, cap,
-                           lc, ray_counter, counters);
+                           deal.lc, ray_counter, counters);
     };
     const bool wide = bvh.wide != 0, stats = counters != nullptr;
     if (opaque && !any && !stats) {
