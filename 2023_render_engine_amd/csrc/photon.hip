@@ -104,9 +104,12 @@ constexpr uint32_t kLdsK = 128;    // k up to this keeps its heap in LDS
 // queries (8, 16, 32: 12.7, 12.2, 13.5 ms).
 constexpr uint32_t kWalkSteps = 4, kParked = 4, kHeapBatch = 8, kHeapRest = 32, kKnnRefill = 16;
 // A search past this many nodes is given up to be finished by a whole
-// wavefront: the mean query visits 600, the queries between clusters 10^4 to
-// 10^5 (1024, 2048, 4096: 14.0, 13.0, 14.1 ms).
-constexpr uint32_t kHeavySteps = 2048;
+// wavefront: with k = 100 the mean query visits 600, the queries between
+// clusters 10^4 to 10^5 (1024, 2048, 4096: 14.0, 13.0, 14.1 ms).  An ordinary
+// search visits more nodes the more photons it is to find: kHeavyPerEntry for
+// each of them (100,000 queries, k = 1024: 217 ms with 2048, 151 with 8 per
+// entry, 160 with 16).
+constexpr uint32_t kHeavySteps = 2048, kHeavyPerEntry = 8;
 // Searches left in a wavefront that it finishes one after the other with all
 // its lanes (2, 4, 8, 16: 13.8, 14.7, 15.9, 29 ms per photon-mapped frame,
 // whose later bounces make a few thousand queries).
@@ -152,18 +155,24 @@ __device__ inline uint32_t spread10(uint32_t v)
 // of those were taken up; and their slots.  A slot is 0 until its query + 1
 // is written, and kHeavyPassed once a taker has been there: a taker that
 // comes before the query is written goes on, and the giver, who sees it, keeps
-// the search.  Nobody waits for anybody.
-constexpr uint32_t kHeavyTail = 1, kHeavyHead = 2, kHeavySlots = 64, kHeavyMax = 4096, kHeavyPassed = 0xffffffffu;
-constexpr uint32_t kClaimWords = kHeavySlots + kHeavyMax;
+// the search.  Nobody waits for anybody.  There is a slot for each query, and
+// no search is given up twice, so the slots never run out: with 4096 of them,
+// 20,000 queries uniform between 16 clusters (k = 100), of which none is
+// ordinary, took 360 ms, most of them walked to the end by their lanes.
+constexpr uint32_t kHeavyTail = 1, kHeavyHead = 2, kHeavySlots = 64, kHeavyPassed = 0xffffffffu;
+inline size_t claim_bytes(uint32_t queries)
+{
+    return (((size_t)kHeavySlots + queries) * sizeof(uint32_t) + 255) & ~(size_t)255;
+}
 constexpr uint32_t kNeverHeavy = 0x80000000u;
 
-__device__ inline uint32_t pop_heavy(uint32_t *claim)
+__device__ inline uint32_t pop_heavy(uint32_t *claim, uint32_t slots)
 {
     uint32_t h = __hip_atomic_load(claim + kHeavyHead, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     for (;;) {
         const uint32_t t = __hip_atomic_load(claim + kHeavyTail, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        if (h >= min(t, kHeavyMax)) return 0;
-        // heads only grow, up to kHeavyMax: a failed exchange means another taker advanced
+        if (h >= min(t, slots)) return 0;
+        // heads only grow, up to the tail: a failed exchange means another taker advanced
         const uint32_t seen = atomicCAS(claim + kHeavyHead, h, h + 1);
         if (seen == h) {
             const uint32_t v = atomicExch(claim + kHeavySlots + h, kHeavyPassed);
@@ -184,8 +193,9 @@ __global__ __launch_bounds__(256) void k_query_morton(const float *q, uint32_t m
                                                       const uint32_t *m_dev, uint32_t *claim)
 {
     const uint32_t i = blockIdx.x * 256 + threadIdx.x;
-    for (uint32_t j = i; j < kClaimWords; j += gridDim.x * 256) claim[j] = 0;
+    if (i < kHeavySlots) claim[i] = 0;
     if (i >= m) return;
+    claim[kHeavySlots + i] = 0;
     if (m_dev && i >= *m_dev) {
         key[i] = 0xffffffffu;
         id[i] = i;
@@ -672,7 +682,7 @@ __global__ __launch_bounds__(kThreads) void k_photon_knn(KnnArgs a)
                 if (!drained) continue;
                 // no query of its own left: one that another wavefront gave up
                 uint32_t give = 0;
-                if (lane == 0) give = pop_heavy(a.claim);
+                if (lane == 0) give = pop_heavy(a.claim, a.m);
                 give = (uint32_t)__builtin_amdgcn_readfirstlane((int)give);
                 if (give == 0) break;
                 begin(lane == 0, give - 1);
@@ -853,7 +863,7 @@ __global__ __launch_bounds__(kThreads) void k_photon_knn(KnnArgs a)
         // Searches that visit far more nodes than the rest are given up, to be
         // started again by the whole wavefront (below) that first runs out
         // of queries: several of them in one wavefront would hold the launch.
-        const bool heavy = walking && steps > kHeavySteps && steps < kNeverHeavy;
+        const bool heavy = walking && steps > max(kHeavySteps, kHeavyPerEntry * a.k) && steps < kNeverHeavy;
         const uint64_t hv = __ballot(heavy);
         if (hv != 0) {
             // the rows' partial results leave this XCD's L2 before another
@@ -864,11 +874,11 @@ __global__ __launch_bounds__(kThreads) void k_photon_knn(KnnArgs a)
             base = (uint32_t)__builtin_amdgcn_readfirstlane((int)base);
             if (heavy) {
                 const uint32_t at = base + (uint32_t)__popcll(hv & ((1ull << lane) - 1ull));
-                if (at < kHeavyMax && atomicExch(a.claim + kHeavySlots + at, q + 1) != kHeavyPassed) {
+                if (at < a.m && atomicExch(a.claim + kHeavySlots + at, q + 1) != kHeavyPassed) {
                     has = walking = make = false;
                     np = 0;
                 } else {
-                    steps = kNeverHeavy;  // no room, or the slot was passed over: goes on here
+                    steps = kNeverHeavy;  // the slot was passed over: goes on here
                 }
             }
         }
@@ -1155,7 +1165,7 @@ static rt_status sort_queries(rt_photon_map *m, const float *queries, uint32_t n
                                                       (uint32_t *)nullptr, (uint32_t *)nullptr, (int)nq, 0, 30,
                                                       stream);
     const size_t ids = ((size_t)nq * sizeof(uint32_t) + 255) & ~(size_t)255;
-    const size_t need = 4 * ids + kClaimWords * sizeof(uint32_t) + sort_bytes;
+    const size_t need = 4 * ids + claim_bytes(nq) + sort_bytes;
     if (e == hipSuccess && need > m->work_bytes) {
         if (m->work) {
             e = hipStreamSynchronize(stream);
@@ -1177,7 +1187,7 @@ static rt_status sort_queries(rt_photon_map *m, const float *queries, uint32_t n
                                                          m->scale[1], m->scale[2], key0, id0, nullptr, (uint32_t *)(w + 4 * ids));
     e = hipGetLastError();
     if (e == hipSuccess)
-        e = hipcub::DeviceRadixSort::SortPairs(w + 4 * ids + kClaimWords * sizeof(uint32_t), sort_bytes, key0, key1, id0, id1, (int)nq, 0, 30, stream);
+        e = hipcub::DeviceRadixSort::SortPairs(w + 4 * ids + claim_bytes(nq), sort_bytes, key0, key1, id0, id1, (int)nq, 0, 30, stream);
     if (e != hipSuccess) {
         set_error(std::string(who) + ": query sort: " + hipGetErrorString(e));
         return RT_ERR_HIP;
@@ -1197,7 +1207,7 @@ static void render_layout(uint32_t cap, uint32_t k, size_t sort_bytes, size_t &i
                           size_t &ib, size_t &gather)
 {
     ids = ((size_t)cap * sizeof(uint32_t) + 255) & ~(size_t)255;
-    work = 4 * ids + kClaimWords * sizeof(uint32_t) + sort_bytes;
+    work = 4 * ids + claim_bytes(cap) + sort_bytes;
     cb = ((size_t)cap * 4 + 255) & ~(size_t)255;
     ib = ((size_t)cap * k * 4 + 255) & ~(size_t)255;
     gather = 2 * cb + 2 * ib;  // counts, indices, distances (the search's slot pool), farthest distances
@@ -1259,7 +1269,7 @@ hipError_t photon_gather_render(rt_photon_map *m, const float *points, const flo
     k_query_morton<<<(cap + 255) / 256, 256, 0, s>>>(points, cap, m->lo[0], m->lo[1], m->lo[2], m->scale[0],
                                                       m->scale[1], m->scale[2], key0, id0, n_dev, (uint32_t *)(w + 4 * ids));
     if ((e = hipGetLastError()) != hipSuccess) return e;
-    if ((e = hipcub::DeviceRadixSort::SortPairs(w + 4 * ids + kClaimWords * sizeof(uint32_t), sort_bytes, key0, key1, id0, id1, (int)cap, 0, 32, s)) !=
+    if ((e = hipcub::DeviceRadixSort::SortPairs(w + 4 * ids + claim_bytes(cap), sort_bytes, key0, key1, id0, id1, (int)cap, 0, 32, s)) !=
         hipSuccess)
         return e;
     uint8_t *gw = (uint8_t *)m->gather;

@@ -214,3 +214,24 @@ def test_long_searches_keep_the_reference_heap_order(rt, gpu_ctx, k):
         assert np.array_equal(got[0], want[0])
         assert np.array_equal(got[1], want[1])
         assert np.array_equal(got[2], want[2])
+
+
+@pytest.mark.parametrize("k", [5, 100, 300, 1024])
+def test_batches_of_long_searches(rt, gpu_ctx, k):
+    """Nearly every query of a batch lies between clusters and visits thousands
+    of nodes, so thousands of searches are given up and taken over; with k =
+    1024 the ordinary queries among them visit nearly as many."""
+    rng = np.random.default_rng(700 + k)
+    c = np.array([[0, 0, 0], [3, 0.2, 0.1], [1.4, 2.5, 0.3], [1.5, 1.2, 2.8]])
+    x = (c[rng.integers(0, 4, 40000)] + rng.normal(0, 0.1, (40000, 3))).astype(np.float32)
+    x = np.unique(x, axis=0)
+    tree = oracle.kd_build(x)[:2]
+    q = (np.array([1.5, 0.9, 0.8]) + rng.normal(0, 0.3, (6000, 3))).astype(np.float32)
+    near = rng.integers(0, 6000, 600)
+    q[near] = x[rng.integers(0, len(x), 600)] + np.float32(0.01)
+    print(f"[photon] batches of long searches k={k}", flush=True)
+    got = gpu_knn(rt, gpu_ctx, x, q, k, 100.0)
+    want = oracle.knn(x, q, k, 100.0, tree=tree)
+    assert np.array_equal(got[0], want[0])
+    assert np.array_equal(got[1], want[1])
+    assert np.array_equal(got[2], want[2])
