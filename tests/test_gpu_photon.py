@@ -235,3 +235,35 @@ def test_batches_of_long_searches(rt, gpu_ctx, k):
     assert np.array_equal(got[0], want[0])
     assert np.array_equal(got[1], want[1])
     assert np.array_equal(got[2], want[2])
+
+
+@pytest.mark.parametrize("k", [1, 2, 3, 4, 6, 7, 8])
+@pytest.mark.parametrize("radius", [900.0, 1e6])
+def test_small_heaps_with_ties(rt, gpu_ctx, k, radius):
+    """Photons in pairs c + v and c - v around centres that are asked for:
+    distances tie in pairs, and which photon stays is the heap's choice.  Up to
+    7 entries the heap takes a photon as soon as the walk meets it, beyond it is
+    parked.  Whole coordinates below 2^24, none of them twice on an axis."""
+    rng = np.random.default_rng(k)
+    c = np.stack(np.meshgrid(*[np.arange(4)] * 3), -1).reshape(-1, 1, 3) * 20000
+    v = rng.integers(-1000, 1000, (len(c), 12, 3))
+    x = np.concatenate([c + v, c - v], 1).reshape(-1, 3) + 100000
+    keep = np.ones(len(x), bool)
+    for a in range(3):
+        keep &= np.isin(np.arange(len(x)), np.unique(x[:, a], return_index=True)[1])
+    half = keep.reshape(len(c), 2, 12)
+    x = x[(half & half[:, ::-1]).reshape(-1)].astype(np.float32)
+    assert len(x) > 500
+    x = x[rng.permutation(len(x))]
+    tree = oracle.kd_build(x)[:2]
+    q = (np.repeat(c.reshape(-1, 3), 10, 0) + 100000).astype(np.float32)
+    q[::10] += rng.integers(-500, 500, (len(c), 3)).astype(np.float32)
+    shape = rng.integers(0, 3, len(x)).astype(np.int32)
+    for sh, qs in ((None, None), (shape, rng.integers(0, 3, len(q)).astype(np.int32))):
+        got = gpu_knn(rt, gpu_ctx, x, q, k, radius, sh, qs)
+        want = oracle.knn(x, q, k, radius, sh, qs, tree=tree)
+        assert np.array_equal(got[0], want[0])
+        for i in range(len(q)):
+            n = want[0][i]
+            assert np.array_equal(got[1][i, :n], want[1][i, :n]), i
+            assert np.array_equal(got[2][i, :n], want[2][i, :n]), i
