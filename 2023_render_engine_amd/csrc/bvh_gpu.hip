@@ -967,8 +967,9 @@ hipError_t build_bvh_device(const float *xyz, uint32_t nv, const uint32_t *idx, 
     }
     if (wide) {
         // level by level from the root, breadth-first numbering, kLevels of them
-        // (each is two launches) before a look at how far it went; num_nodes2
-        // bounds any level's frontier
+        // (each is two launches) before a look at how far it went, and no more
+        // than the kept two-wide tree has (a wide level takes one or more of
+        // them); num_nodes2 bounds any level's frontier
         const uint32_t cap4 = out.num_nodes2;
         const unsigned grid = std::min(blocks(cap4), kCollapseBlocks);
         size_t off = 0;
@@ -984,11 +985,12 @@ hipError_t build_bvh_device(const float *xyz, uint32_t nv, const uint32_t *idx, 
         hipLaunchKernelGGL(k_collapse4_begin, dim3(1), dim3(64), 0, s, front[0], st);
         uint32_t level = 0;
         for (bool more = true; more;) {
-            if (level + kLevels > kMaxLevels) {
+            const uint32_t upto = std::min({level + kLevels, out.max_depth, kMaxLevels});
+            if (level >= upto) {
                 err = "rt_bvh_build_device: four-wide tree deeper than its two-wide tree can be";
                 return hipErrorUnknown;
             }
-            for (uint32_t k = 0; k < kLevels; ++k, ++level) {
+            for (; level < upto; ++level) {
                 const uint32_t cur = level & 1u;
                 hipLaunchKernelGGL(k_collapse4_count, dim3(grid), dim3(kBB), 0, s, out.nodes2, front[cur],
                                    st->level + level, cnt, bsum);
