@@ -429,9 +429,9 @@ struct Collapser {
             for (int i = 1; i < nk; ++i) p = std::min(p, kids[i].lo[a]);
             double ext = 0.0;
             for (int i = 0; i < nk; ++i) ext = std::max(ext, (double)kids[i].hi[a] - (double)p);
-            const int e = scale_exponent(ext);
+            const int e = std::min(scale_exponent(ext), kMaxScaleExp);
             const double sc = std::ldexp(1.0, e);
-            n.origin[a] = p;
+            n.origin[a] = ext > 255.0 * sc ? std::nanf("") : p;
             meta |= (uint32_t)(e + 127) << (8 * a);
             uint32_t qlo = 0, qhi = 0;
             for (int i = 0; i < nk; ++i) {

@@ -715,9 +715,9 @@ __device__ void collapse_entry(const Node2 *n2, const uint2 *front, uint32_t f, 
 #pragma unroll
         for (uint32_t i = 0; i < 4; ++i)
             if (i < nk) ext = fmax(ext, (double)kids[i].hi[a] - (double)p);
-        const int e = scale_exponent(ext);
+        const int e = min(scale_exponent(ext), kMaxScaleExp);
         const double sc = ldexp(1.0, e), inv = ldexp(1.0, -e);  // x * inv is x / sc exactly
-        n.origin[a] = p;
+        n.origin[a] = ext > 255.0 * sc ? __builtin_nanf("") : p;
         meta |= (uint32_t)(e + 127) << (8 * a);
         uint32_t qlo = 0, qhi = 0;
 #pragma unroll

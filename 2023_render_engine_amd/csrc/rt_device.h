@@ -132,10 +132,17 @@ __device__ __forceinline__ bool tri_intersects(const TriRay &r, const float4 a, 
     return true;
 }
 
-// Slab-test constants.  A direction component below 1e-22 is replaced by
-// +-1e-22, so no 0 * inf NaN can arise and a node's scale times 2^24 / d stays
-// finite (scales up to 10^9); the padded boxes keep the test conservative.
-constexpr float kMinDir = 1e-22f;
+// Slab-test constants.  A direction component below 1e-16 in size is replaced
+// by +-1e-16, so no 0 * inf NaN can arise and a node's scale (at most
+// 2^kMaxScaleExp) times 2^24 / d stays finite.  The boxes stay conservative,
+// also for short directions: the triangle test rejects t <= deltaT, and as
+// deltaT >= 1.5 error_bound(5) maxZt^2 / min(maxXt, maxYt), an accepted hit at
+// depth L on a triangle of size s has L < 4.4e6 m s, m the largest direction
+// component.  The replacement moves the ray by at most 1e-16 L / m < 5e-10 s at
+// that depth, and the boxes are padded by 2^-19 s or more.  From outside the
+// padded box L >= 2^-19 s, so m > 4e-13 is not replaced itself; from inside,
+// the slab test holds for any direction.
+constexpr float kMinDir = 1e-16f;
 struct BoxRay {
     float ix, iy, iz;     // 1 / d
     float oix, oiy, oiz;  // o / d

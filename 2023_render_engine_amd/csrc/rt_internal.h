@@ -56,6 +56,10 @@ inline int32_t encode_leaf(uint32_t first, uint32_t count)
 // An unused slot holds an empty box (lo byte 255, hi byte 0) and a leaf
 // reference to the tree's degenerate sentinel triangle.
 // Child box i along x: [origin.x + lo_x[i] * sx, origin.x + hi_x[i] * sx].
+// Children that span more than 255 * 2^kMaxScaleExp (3e17) along an axis are
+// not bounded on it: the origin is NaN there, and the slab test passes over NaN
+// distances.  At that size the products of the triangle test overflow but for
+// triangles much smaller than the span.
 struct alignas(64) Node4 {
     float origin[3];
     uint32_t meta;
@@ -63,6 +67,7 @@ struct alignas(64) Node4 {
     uint32_t q[8];
 };
 static_assert(sizeof(Node4) == 64, "wide node must be one cache line");
+constexpr int kMaxScaleExp = 50;
 
 struct HostBvh {
     std::vector<Node2> nodes;

@@ -260,3 +260,46 @@ def test_small_launches_and_axis_parallel_rays(rt, orc, gpu_ctx, n, scale):
     occ = bvh.trace_any(*to_dev(rays), torch.from_numpy(tmax).cuda())
     torch.cuda.synchronize()
     assert np.array_equal(occ.cpu().numpy()[clean].astype(bool), bp[clean] >= 0)
+
+
+@pytest.mark.parametrize("device", [False, True])
+@pytest.mark.parametrize("case", ["large", "far vertex", "short 1e-5", "short 1e-12", "short 1e-23"])
+def test_extreme_scenes_and_directions(rt, orc, gpu_ctx, case, device):
+    """Axis-parallel rays in a scene 10^12 across (the slab distances of a zero
+    direction component must not overflow), a scene with one vertex at 10^34
+    (nodes whose scale leaves the float range), and directions of length 10^-5,
+    10^-12 and 10^-23: ids and distances equal brute force on unambiguous
+    rays."""
+    n = 600
+    xyz, idx = rt.gen_soup(400, seed=9, edge_mu=0.2)
+    rays = [a[:n].copy() for a in rt.gen_rays(1, 1, n_incoherent=n, seed=4)]
+    for k in range(0, n, 2):
+        d = np.zeros(3, np.float32)
+        d[(k // 2) % 3] = 1.0 if k % 4 else -1.0
+        for c in range(3):
+            rays[3 + c][k] = d[c]
+    if case == "large":
+        xyz = (xyz * np.float32(1e12)).astype(np.float32)
+        for c in range(3):
+            rays[c] = (rays[c] * np.float32(1e12)).astype(np.float32)
+    elif case == "far vertex":
+        xyz = np.concatenate([xyz, np.float32([[0.2, 0.3, 5.0], [0.4, 0.1, 6.0], [1e34, -2e33, 3e33]])])
+        idx = np.concatenate([idx, np.uint32([[len(xyz) - 3, len(xyz) - 2, len(xyz) - 1]])])
+    else:
+        for c in range(3, 6):
+            rays[c] = (rays[c].astype(np.float64) * float(case.split()[1])).astype(np.float32)
+    if device:
+        bvh = rt.Bvh.from_device(gpu_ctx, torch.from_numpy(xyz).cuda(), torch.from_numpy(idx.view(np.int32)).cuda())
+    else:
+        bvh = rt.Bvh(gpu_ctx, xyz, idx)
+    prim, t = bvh.trace_closest(*to_dev(rays))
+    bp, bt, fl = orc.brute_trace(xyz, idx, rays)
+    clean = fl == 0
+    assert clean.mean() > 0.5
+    # the triangle test itself rejects every hit of the two shorter ones
+    assert (bp >= 0).sum() > 100 or case in ("short 1e-12", "short 1e-23")
+    torch.cuda.synchronize()
+    prim, t = prim.cpu().numpy(), t.cpu().numpy()
+    assert np.array_equal(prim[clean], bp[clean])
+    assert np.array_equal(t[clean], bt[clean])
+    bvh.close()
