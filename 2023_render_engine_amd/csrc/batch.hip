@@ -64,7 +64,7 @@ struct rt_batch {
     std::vector<rt_scene *> scenes;
     std::vector<rt::SceneDev> host_table;   // as uploaded (seeds included)
     std::vector<uint32_t> npix;
-    uint32_t stack_cap = 0, max_lights = 1;
+    uint32_t stack_cap = 0, max_lights = 1, max_area = 0;
     uint64_t paths_per_sample = 0;           // sum of pixels
     rt::SceneDev *d_table = nullptr;
     void *d_nodes = nullptr, *d_tris = nullptr;  // the scenes' trees, pooled
@@ -353,6 +353,7 @@ rt_status rt_batch_create(rt_ctx *ctx, rt_scene *const *scenes, uint32_t n, rt_b
             return RT_ERR_INVALID;
         }
         b->max_lights = std::max(b->max_lights, d.nlights);
+        b->max_area = std::max(b->max_area, d.nlights - d.npl);
         b->paths_per_sample += (uint64_t)d.cam.width * d.cam.height;
     }
     if (b->stack_cap > rt::kMaxTraversalStack) {
@@ -436,7 +437,7 @@ rt_status rt_batch_render(rt_batch *b, const rt_batch_opts *opts, const uint32_t
     const uint64_t total = b->paths_per_sample * opts->spp;
     const uint32_t P = wave_size(b, *opts, total);
     const uint32_t grid = opts->grid ? opts->grid : (b->tuned_grid ? b->tuned_grid : 2048);
-    st = rt::ensure_wave_buffers(b->wb, P, b->max_lights, "rt_batch_render");
+    st = rt::ensure_wave_buffers(b->wb, P, b->max_lights, b->max_area, "rt_batch_render");
     const uint64_t chunk = opts->chunk_paths ? opts->chunk_paths : rt::kChunkPaths;
     if (st == RT_OK) st = rt::ensure_result_buffer(b->wb, std::min<uint64_t>(total, chunk), "rt_batch_render");
     if (st != RT_OK) return st;
@@ -511,7 +512,7 @@ rt_status rt_batch_autotune(rt_batch *b, const rt_batch_opts *opts, rt_tune_entr
     if (result == RT_OK) result = upload_bases(b, o.spp, s);
     for (uint32_t P : caps) {
         if (result != RT_OK) break;
-        result = rt::ensure_wave_buffers(b->wb, P, b->max_lights, "rt_batch_autotune");
+        result = rt::ensure_wave_buffers(b->wb, P, b->max_lights, b->max_area, "rt_batch_autotune");
         if (result == RT_OK)
             result = rt::ensure_result_buffer(b->wb, std::min<uint64_t>(total, rt::kChunkPaths), "rt_batch_autotune");
         for (uint32_t gsz : grids) {

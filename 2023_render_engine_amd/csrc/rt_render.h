@@ -129,7 +129,7 @@ struct PathsDev {
 struct ShadowDev {
     uint32_t *ray;              // vertex within the stripe << 5 | light slot
     float4 *org;                // [stripe][vertex]: origin, vertex x | vertex yz, path slot, scene (batches)
-    float4 *area;               // [area light][stripe][vertex]: direction, tMax
+    float4 *area;               // [area light][stripe][vertex]: direction, tMax (none without area lights)
 };
 
 struct QueuesDev {

@@ -12,6 +12,7 @@ namespace rt {
 struct WaveBuffers {
     uint32_t capacity = 0;    // path slots
     uint32_t cap_lights = 0;  // light slots per path
+    uint32_t cap_area = 0;    // area lights among them
     void *arena = nullptr;
     PathsDev paths{};
     ShadowDev shadow{};
@@ -21,10 +22,10 @@ struct WaveBuffers {
     uint32_t *host_counters = nullptr;  // pinned, kNumCounters words
 };
 
-// Grows `w` to at least P path slots with NL light slots each (one
-// allocation, 256-byte aligned pieces).  `who` names the caller in the
-// error text.
-rt_status ensure_wave_buffers(WaveBuffers &w, uint32_t P, uint32_t NL, const char *who);
+// Grows `w` to at least P path slots with NL light slots each, `area` of them
+// area lights' (one allocation, 256-byte aligned pieces).  `who` names the
+// caller in the error text.
+rt_status ensure_wave_buffers(WaveBuffers &w, uint32_t P, uint32_t NL, uint32_t area, const char *who);
 // Grows the chunk result buffer to R paths.
 rt_status ensure_result_buffer(WaveBuffers &w, uint64_t R, const char *who);
 void free_wave_buffers(WaveBuffers &w);

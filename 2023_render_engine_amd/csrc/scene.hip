@@ -319,10 +319,10 @@ static rt_status ensure_photon_rows(rt_scene *s, uint32_t rows, PhotonLaunch &ph
 
 // One allocation for all wavefront buffers, carved in 256-byte aligned
 // pieces: paths (SoA), shadow queue (capacity * lights entries), queues.
-rt_status ensure_wave_buffers(WaveBuffers &w, uint32_t P, uint32_t NL, const char *who)
+rt_status ensure_wave_buffers(WaveBuffers &w, uint32_t P, uint32_t NL, uint32_t area, const char *who)
 {
     NL = std::max<uint32_t>(1, NL);
-    if (w.capacity >= P && w.cap_lights >= NL) return RT_OK;
+    if (w.capacity >= P && w.cap_lights >= NL && w.cap_area >= area) return RT_OK;
     if (w.arena) (void)hipFree(w.arena);
     w.arena = nullptr;
     w.capacity = 0;
@@ -350,7 +350,7 @@ rt_status ensure_wave_buffers(WaveBuffers &w, uint32_t P, uint32_t NL, const cha
     ShadowDev &sh = w.shadow;
     add((void **)&sh.ray, SQ * 4);
     add((void **)&sh.org, (size_t)P * 2 * sizeof(float4));
-    add((void **)&sh.area, SQ * sizeof(float4));
+    add((void **)&sh.area, (size_t)P * area * sizeof(float4));
     QueuesDev &q = w.queues;
     add((void **)&q.active[0], (size_t)P * 4);
     add((void **)&q.active[1], (size_t)P * 4);
@@ -371,6 +371,7 @@ rt_status ensure_wave_buffers(WaveBuffers &w, uint32_t P, uint32_t NL, const cha
     w.arena = base;
     w.capacity = P;
     w.cap_lights = NL;
+    w.cap_area = area;
     return RT_OK;
 }
 
@@ -406,9 +407,11 @@ rt_status fill_stats(rt_render_stats &st, const unsigned long long *counts, Kern
 
 static rt_status ensure_buffers(rt_scene *s, uint32_t P, const char *who)
 {
-    if (s->wb.capacity >= P && s->wb.cap_lights >= std::max<uint32_t>(1, s->dev.nlights)) return RT_OK;
-    free_arena(s);  // the cache scratch is sized to the wave capacity too
-    return ensure_wave_buffers(s->wb, P, s->dev.nlights, who);
+    const uint32_t area = s->dev.nlights - s->dev.npl;
+    if (s->wb.capacity >= P && s->wb.cap_lights >= std::max<uint32_t>(1, s->dev.nlights) && s->wb.cap_area >= area)
+        return RT_OK;
+    free_arena(s);  // the photon rows are sized to the wave capacity too
+    return ensure_wave_buffers(s->wb, P, s->dev.nlights, area, who);
 }
 
 }  // namespace rt
