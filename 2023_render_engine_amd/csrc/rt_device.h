@@ -413,7 +413,9 @@ __device__ __forceinline__ float byte_half(const BytePairs &b, int i)
 
 // Pushes ref[3], ref[2], ref[1] where their key is a hit.  Every entry is
 // written at the stack's end and counted or not, so the write past the last
-// entry needs a place: the stack holds one more than the tree can need.
+// entry needs a place: the stack holds one more than the tree can need.  The
+// bound is the tree's own (the builders compute it exactly); nothing is checked
+// here.
 template <class S>
 __device__ __forceinline__ void stack_push3(const S &st, int &sp, const int32_t ref[4], const uint32_t key[4])
 {
@@ -435,7 +437,7 @@ __device__ __forceinline__ void stack_push3(const S &st, int &sp, const int32_t 
 
 template <bool ANY, bool STATS, class Stack, bool OPAQUE = false>
 __device__ __forceinline__ bool trav_step4(TravState &s, const float4 *__restrict__ nodes,
-                                           const float4 *__restrict__ tris, const Stack &stack, int cap,
+                                           const float4 *__restrict__ tris, const Stack &stack,
                                            uint32_t leaf_batch, uint32_t &n_node, uint32_t &n_tri)
 {
     // kNodeSteps interior-node visits (each followed by parking a reached
@@ -539,7 +541,7 @@ __device__ __forceinline__ bool trav_step_any(TravState &s, const float4 *__rest
                                               uint32_t leaf_batch, uint32_t &n_node, uint32_t &n_tri)
 {
     if constexpr (WIDE)
-        return trav_step4<ANY, STATS, Stack, OPAQUE>(s, nodes, tris, stack, cap, leaf_batch, n_node, n_tri);
+        return trav_step4<ANY, STATS, Stack, OPAQUE>(s, nodes, tris, stack, leaf_batch, n_node, n_tri);
     else return trav_step<ANY, STATS, Stack, OPAQUE>(s, nodes, tris, stack, cap, n_node, n_tri);
 }
 

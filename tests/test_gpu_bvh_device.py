@@ -6,6 +6,7 @@ are bitwise equal and the reported figures match; traces on the device-built
 tree agree with brute force on every unambiguous ray; transparency and the
 error paths work as on the host-built tree."""
 import ctypes as C
+import importlib
 
 import numpy as np
 import pytest
@@ -187,3 +188,88 @@ def test_full_size_device_build(rt, orc, gpu_ctx):
         _, _, fk = orc.brute_trace(xyz, idx, [a[dk] for a in rays], nthreads=16)
         assert np.all(fk != 0), dk[fk == 0][:10]
     bvh.close()
+
+
+def deep_chain(n):
+    """Thirty steps towards a corner, each with four triangles larger than all
+    that follows, and n equal ones at its end: the wide nodes open the steps'
+    triangles, so up to three entries are pending per level."""
+    rng = np.random.default_rng(1)
+    out = []
+    for k in range(10):
+        for a in range(3):
+            p = 0.75 * 2.0**-k * np.eye(3)[a]
+            for j in range(4):
+                t = rng.uniform(-1, 1, (3, 3))
+                lo, hi = t.min(0), t.max(0)
+                t = (t - (lo + hi) / 2) / (hi - lo) * 2  # the cube [-1, 1]^3 bounds it
+                out.append(p + 1.5 * 2.0**-(k + a / 3) * (1 + 0.02 * j) * t)
+    s = np.array([[0, 0, 0], [1, 0, 0], [0, 1, 1]]) * 2.0**-13
+    out += [s] * n + [1 + s]
+    xyz = np.array(out).astype(np.float32).reshape(-1, 3)
+    return xyz, np.arange(xyz.shape[0], dtype=np.uint32).reshape(-1, 3)
+
+
+def corner_rays(n, seed):
+    """Rays that pass close by the corner from near and far."""
+    rng = np.random.default_rng(seed)
+    o = rng.normal(0, 1e-4, (n, 3))
+    d = rng.normal(0, 1, (n, 3))
+    d /= np.linalg.norm(d, axis=1)[:, None]
+    o -= d * rng.choice([0, 1e-3, 3.0], (n, 1))
+    return [np.ascontiguousarray(v[:, c].astype(np.float32)) for v in (o, d) for c in range(3)]
+
+
+@pytest.mark.parametrize("n,cap", [(1, 92), (4096, 124), (16381, 128)])
+def test_traversal_stack_bound(rt, orc, gpu_ctx, n, cap):
+    """Trees that need a deep stack, up to the largest that is accepted (129
+    entries of every lane in LDS with the mark at the bottom).  The restated
+    walk's pending entries stay within the bound, and the kernels' hits are
+    its hits: distances, and ids where no equal triangle ties."""
+    xyz, idx = deep_chain(n)
+    bvh = device_bvh(rt, gpu_ctx, xyz, idx, max_leaf=1)
+    assert bvh.info().stack_cap == cap
+    rays = corner_rays(5000, n)
+    p2, t2, _, _, msp = orc.bvh4_trace(bvh.export4(), bvh.export()[1], rays)
+    print(f"[bvh device] deep chain n={n}: {msp} entries of {cap}", flush=True)
+    assert 80 <= msp <= cap - 1  # the rays use most of it
+    prim, t = bvh.trace_closest(*to_dev(rays))
+    occ = bvh.trace_any(*to_dev(rays), torch.full((5000,), 10.0, device="cuda"))
+    torch.cuda.synchronize()
+    prim, t, occ = prim.cpu().numpy(), t.cpu().numpy(), occ.cpu().numpy().astype(bool)
+    assert np.array_equal(t, t2)
+    steps = 120
+    same = (p2 < steps) | (prim < steps)
+    assert np.array_equal(prim[same], p2[same]) and np.all((prim >= steps) == (p2 >= steps))
+    assert np.array_equal(occ, (p2 >= 0) & (t2 <= 10.0))
+    bvh.close()
+    # one entry more is refused
+    if cap == 128:
+        with pytest.raises(rt.RtError):
+            device_bvh(rt, gpu_ctx, *deep_chain(n + 2), max_leaf=1)
+
+
+def test_deep_stack_in_the_renderer(rt, gpu_ctx):
+    """The path tracer keeps 24 stack entries in LDS and the rest in private
+    memory: a scene whose tree needs 124 gives the image of the same scene
+    under a host-built tree, on (almost) every pixel."""
+    scenes = importlib.import_module("2023_render_engine_amd.scenes")
+    xyz, idx = deep_chain(4096)
+    d = scenes.cornell(width=64, height=64, spp=4)
+    d.xyz, d.idx, d.tri_mat = xyz, idx, (np.arange(len(idx)) % 3).astype(np.uint32)
+    d.tri_mat[120:] = 0
+    d.spheres, d.lights = [], [((-1.7, 0.4, 0.3), (1, 1, 1), 10.0), ((-1.5, -0.5, 0.6), (1, 1, 1), 10.0)]
+    out = []
+    for kw in (dict(), dict(bvh_on_device=True, bvh_max_leaf=1), dict(bvh_on_device=True, bvh_max_leaf=1, bvh_width=2)):
+        sc = rt.Scene(gpu_ctx, d, **kw)
+        film = sc.new_film()
+        sc.render(film)
+        torch.cuda.synchronize()
+        out.append((film[0].cpu().numpy().reshape(-1, 3), film[1].cpu().numpy()))
+        sc.close()
+    assert out[0][0].mean() > 0
+    for a, n in out[1:]:
+        same = np.all(a == out[0][0], axis=1)
+        print(f"[bvh device] deep stack in the renderer: {same.mean():.4f} of pixels equal", flush=True)
+        assert np.array_equal(n, out[0][1])
+        assert same.mean() >= 0.99
