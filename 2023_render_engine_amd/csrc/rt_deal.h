@@ -64,13 +64,12 @@ RT_HD uint32_t deal_refill(uint32_t width) { return (width * kRefillLanes) >> 6;
 static_assert((kMinWidth * kRefillLanes) >> 6 >= 1, "kRefillLanes of 64 lanes is at least one of kMinWidth lanes");
 
 // Items of the next claim: `left` items of the stripe over its 2^wlog
-// wavefronts, between kClaimMin and kClaimChunk; a narrow wavefront claims what
-// it can start at once.
+// wavefronts, between kClaimMin (what a narrow wavefront can start at once,
+// if that is less) and kClaimChunk.
 RT_HD uint32_t deal_claim(uint32_t left, uint32_t wlog, uint32_t width)
 {
-    if (width < 64u) return width;
-    const uint32_t k = left >> wlog;
-    return k < kClaimMin ? kClaimMin : (k > kClaimChunk ? kClaimChunk : k);
+    const uint32_t k = left >> wlog, least = width < kClaimMin ? width : kClaimMin;
+    return k < least ? least : (k > kClaimChunk ? kClaimChunk : k);
 }
 
 // A ray batch: dealt to the stripes in chunks of 2^lc consecutive rays (chunk
@@ -114,8 +113,10 @@ inline RayDeal ray_deal(uint32_t n, uint32_t most)
     const uint64_t chunks = ((uint64_t)n + (1u << d.lc) - 1) >> d.lc;
     uint64_t blocks = chunks;  // one chunk per stripe, or none
     if (chunks > kStripes || d.lc > 2) {
+        // (a power of two per stripe, so that a claim's share is what one wavefront starts)
         const uint64_t rays = ((chunks + kStripes - 1) / kStripes) << d.lc;  // of the fullest stripe
-        blocks = kStripes * ((rays + kLanes - 1) / kLanes);
+        for (blocks = kStripes; blocks / kStripes * kLanes < rays; blocks *= 2) {
+        }
     }
     // kWidthWaves wavefronts take up to 64 rays each in one turn; more rays are
     // taken by as many wavefronts as the chip holds
