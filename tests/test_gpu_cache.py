@@ -110,19 +110,44 @@ def test_online_training_fits_a_smooth_field(rt, gpu_ctx):
     cache.close()
 
 
+def last_cells(levels, log2_table, base, scale):
+    """Grid features that are zero but for the last entries of every level: the
+    last table entries of a hashed one, the last row of cells of a dense one."""
+    g = np.zeros((levels, 1 << log2_table, 2), np.float32)
+    for l in range(levels):
+        res = int(np.floor(base * float(np.float32(scale)) ** l))
+        dense = (res + 1) ** 3 <= 1 << log2_table
+        end = (res + 1) ** 3 if dense else 1 << log2_table
+        k = res + 1 if dense else 2
+        g[l, end - k:end] = np.random.default_rng(12 + l).uniform(2, 4, (k, 2))
+    return g.reshape(-1)
+
+
 @pytest.mark.parametrize("levels,log2_table,base,scale", [(1, 8, 2, 1.0), (3, 9, 7, 1.7), (5, 12, 4, 2.0), (16, 10, 16, 1.38)])
 @pytest.mark.parametrize("n", [1, 15, 16, 17, 63, 64, 65, 1000, 70001])
-def test_query_sizes_and_level_counts(rt, gpu_ctx, orc, levels, log2_table, base, scale, n):
+@pytest.mark.parametrize("last", [False, True])
+def test_query_sizes_and_level_counts(rt, gpu_ctx, orc, levels, log2_table, base, scale, n, last):
     """Strips of 16 rows with remainders, level counts that end inside a
     feature tile, dense levels that fill their table (res 7 and 512 entries),
-    positions on the box's faces (the last cell's clamped corners)."""
+    positions on the box's faces (the last cell's clamped corners); with
+    `last`, only the last entries of a level are not zero and most rows lie at
+    the far corner, so that a wrong half of a pair load there is the answer.
+
+    The oracle rounds at the same places, so answers agree to float rounding
+    but for a row in which a sum rounds to the other BF16 neighbour (2^-8 of
+    one of 64 activations; 8.5e-4 of 0.19 measured at most).  Such rows are rare:
+    an RMS of 2e-5 of 0.067 at most.  The last entry of each level zeroed moves the
+    answers by an RMS of 8e-4 to 3e-3, with `last` by 2e-3 to 0.1."""
     cache = rt.RadianceCache(gpu_ctx, (0, 0, 0), (1, 1, 1), levels=levels, log2_table=log2_table, base_res=base,
                              per_level_scale=scale, batch=256, seed=3)
     cfg = orc.cache_cfg(levels, log2_table, base, scale, (0, 0, 0), (1, 1, 1))
     mlp, grid = cache.get_params()
-    grid = np.random.default_rng(11).uniform(-0.5, 0.5, grid.shape).astype(np.float32)
+    grid = (last_cells(levels, log2_table, base, scale) if last
+            else np.random.default_rng(11).uniform(-0.5, 0.5, grid.shape).astype(np.float32))
     cache.set_params(mlp, grid)
     rec = records(n, 1)
+    if last:
+        rec[:, :3] = np.where(np.random.default_rng(3).random((n, 3)) < 0.5, 1.0, 1.0 - 0.1 * rec[:, :3])
     rec[:: 7, 0] = 1.0
     rec[3:: 7, 1] = 0.0
     rec[5:: 7, 2] = 1.0
@@ -132,7 +157,9 @@ def test_query_sizes_and_level_counts(rt, gpu_ctx, orc, levels, log2_table, base
     ref = orc.cache_loss_grad(cfg, mlp, grid, rec[at], np.zeros((m, 3), np.float32), emulate_bf16=True,
                               want_grad=False)[3]
     ref = np.maximum(ref, 0)
-    assert np.max(np.abs(y[at] - ref)) <= 1e-2 * max(1.0, np.max(np.abs(ref)))
+    err = np.abs(y[at] - ref)
+    assert np.max(err) <= 1e-2 * np.max(ref)
+    assert np.sqrt(np.mean(err ** 2)) <= 1e-3 * np.sqrt(np.mean(ref ** 2))
     cache.close()
 
 
