@@ -18,9 +18,11 @@ same rays, run on the host's cores.
 from __future__ import annotations
 
 import argparse
+import hashlib
 import importlib
 import json
 import os
+import re
 import sys
 import time
 
@@ -33,6 +35,29 @@ HBM_PEAK_GBS = 8000.0
 
 def log(msg):
     print(f"[bench] {msg}", file=sys.stderr, flush=True)
+
+
+def sources_sha16(files) -> str:
+    """Hash of the library sources `files` without comments and white space."""
+    h = hashlib.sha256()
+    for f in files:
+        with open(os.path.join(ROOT, "2023_render_engine_amd", "csrc", f)) as src:
+            text = re.sub(r"//[^\n]*|/\*.*?\*/", "", src.read(), flags=re.S)
+        h.update(re.sub(r"\s+", "", text).encode())
+    return h.hexdigest()[:16]
+
+
+def load_profile(name):
+    """The committed profile `name`, or None when there is none or the kernels
+    that it was taken on have changed since (its "sources" name the files
+    and their hash)."""
+    try:
+        with open(os.path.join(ROOT, "profiles", name)) as f:
+            d = json.load(f)
+        src = d["sources"]
+        return d if sources_sha16(src["files"]) == src["sha16"] else None
+    except (OSError, ValueError, KeyError):
+        return None
 
 
 def cpu_threads() -> int:
@@ -140,14 +165,11 @@ def run_c1(args):
 
     achieved = alg_bytes / (k_avg / 1e3) / 1e9
     # HBM traffic and shader counters from the committed profiles of this
-    # workload, used only while they describe it (same algorithmic bytes per
-    # launch within 1 %: the same rays, tree and visit counts)
+    # workload, used only while they describe it (same kernel sources; same
+    # algorithmic bytes per launch within 1 %: the same rays, tree and visits)
     def profile(name):
-        try:
-            d = json.load(open(os.path.join(ROOT, "profiles", name)))
-        except (OSError, ValueError):
-            return None
-        ref = d.get("algorithmic_bytes_per_launch") or 0
+        d = load_profile(name)
+        ref = (d or {}).get("algorithmic_bytes_per_launch") or 0
         return d if ref > 0 and abs(alg_bytes - ref) <= 0.01 * ref else None
     pmc = profile(f"c1_trace_closest_bvh{args.width}_hbm_traffic.json")
     traffic = pmc.get("hbm_bytes_per_launch") if pmc else None
@@ -185,8 +207,8 @@ def run_c1(args):
             "valu": valu,
             "note": ("achieved = 36 B per ray + 64 B per node visit + 48 B per triangle test (counted by the "
                      "kernel's counting variant) / the kernel's HIP-event time; traffic and valu come from the "
-                     "committed FETCH_SIZE / WRITE_SIZE and SQ profiles of this workload (null when the run's "
-                     "algorithmic bytes differ from theirs)"),
+                     "committed FETCH_SIZE / WRITE_SIZE and SQ profiles of this workload (null when the kernel's "
+                     "sources have changed since or the run's algorithmic bytes differ from theirs)"),
         },
         "kernel_ms": round(k_avg, 3),
         "mrays_coherent": split["coherent"],
@@ -217,16 +239,13 @@ DEFAULT_WAVE = 1 << 24
 def measured_traffic(profile, kernel, alg_bytes, field="hbm_bytes_per_frame", wave=None):
     """HBM bytes per frame of `kernel` (or another field of its entry, such
     as its shader counters) from a committed FETCH_SIZE / WRITE_SIZE profile
-    (copy-scaled), or None when there is none or it was taken on another
-    workload (its algorithmic bytes per frame differ from this run's by more
-    than 1 %, or its wave size, when given, is not this run's)."""
-    if not profile:
-        return None
-    path = os.path.join(ROOT, "profiles", profile)
-    try:
-        d = json.load(open(path))
-        k = d["kernels"][kernel]
-    except (OSError, ValueError, KeyError):
+    (copy-scaled), or None when there is none or it was taken on other
+    kernels or another workload (its algorithmic bytes per frame differ from
+    this run's by more than 1 %, or its wave size, when given, is not this
+    run's)."""
+    d = load_profile(profile) if profile else None
+    k = (d or {}).get("kernels", {}).get(kernel)
+    if k is None:
         return None
     if wave is not None and d.get("path_capacity") != wave:
         return None
@@ -699,12 +718,8 @@ def run_film(args):
     bytes_per_call = 51 * npix
     gbs = bytes_per_call / (call_ms * 1e-3) / 1e9
     traffic = None
-    pmc_path = os.path.join(ROOT, "profiles", "film_tonemap_1080p_hbm_traffic.json")
-    if mode == "gammaClamp" and os.path.exists(pmc_path):
-        try:
-            traffic = json.load(open(pmc_path)).get("hbm_bytes_per_call")
-        except (OSError, ValueError):
-            traffic = None
+    if mode == "gammaClamp":
+        traffic = (load_profile("film_tonemap_1080p_hbm_traffic.json") or {}).get("hbm_bytes_per_call")
     res = {
         "metric": "film tone mapping + BMP packing", "value": round(npix * args.steps / wall / 1e6, 1),
         "unit": "Mpixels/s", "n_gpus": 1, "steps": args.steps, "warmup": args.warmup,
