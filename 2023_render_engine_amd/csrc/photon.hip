@@ -24,8 +24,9 @@
 // wavefront's chain of dependent steps (node loads, LDS reads, branches) is
 // the time.  Per wavefront the walk and the heap steps are therefore run
 // apart: a lane parks the photons it meets and walks on with the radius it
-// knows, and the heap step runs once many lanes have something parked.  That
-// leaves the result and its order as they are: the walk with an older, larger
+// knows, and the heap step runs once many lanes have something parked (up to
+// k = 7, whose step is cheap, they stay together).  That leaves the result and
+// its order as they are: the walk with an older, larger
 // radius meets the same photons in the same order and some more; every photon
 // of a subtree that the exact walk passes over is at least as far as the
 // subtree's plane, which was not below the radius (rounding keeps that order),
@@ -387,7 +388,7 @@ __device__ inline void lds_heap_adjust(const LdsHeap &h, uint32_t top, uint32_t 
         }
 }
 
-// The heap steps are calls: inlined at their three uses they made a 100 KB
+// The heap steps are calls: inlined at their uses (three of each) they made a 100 KB
 // kernel, more than the instruction cache holds (6200 cycles per heap step;
 // 2450 as a call without branches).  Each works on the calling lane's LDS
 // column.

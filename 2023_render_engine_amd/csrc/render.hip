@@ -857,9 +857,9 @@ __device__ __forceinline__ void shade_class(const SceneDev &sc0, const BatchDev 
 // All five classes in one launch: workgroup b serves stripe b % kStripes and
 // class b / kStripes % 5, so a wavefront still runs one material.  The
 // classes overlap, which is worth more than each one's own register count
-// (154 for GGX): against five launches the preview frame (333x187, 1 spp)
-// takes 1.40 instead of 1.69 ms, the Cornell box (256x256, 16 spp) 1.68
-// instead of 1.85, a 1080p frame of 64 spp 254.6 instead of 266.6.
+// (154 for GGX): of the time with five launches the preview frame (333x187, 1
+// spp) takes 0.83, the Cornell box (256x256, 16 spp) 0.91, a 1080p frame of 64
+// spp 0.955 (each pair timed in one run).
 template <bool B>
 __global__ __launch_bounds__(kBlock) void k_shade(SceneDev sc0, BatchDev bt, PathsDev p, ShadowDev sh, QueuesDev q,
                                                   WaveParams wp, uint32_t cur)
@@ -1236,8 +1236,8 @@ hipError_t chunk_iterate(const ChunkLaunch &c, const WaveParams &wp, uint32_t it
         else cnt ? go(k_connect<false, false, true>) : go(k_connect<false, false, false>);
     };
     // workgroups per class and stripe: enough for every item of a small wave, at
-    // most 256 (1080p frame at 16, 32, 64, 256 and 2048: 262.6, 257.2, 254.3,
-    // 251.1, 254.5 ms), scaled with the grid option
+    // most 256 (a 1080p frame with 16, 32, 64 and 2048 takes 1.046, 1.024, 1.013
+    // and 1.014 of its time), scaled with the grid option
     const uint32_t most = std::max(1u, (wp.grid ? wp.grid : (uint32_t)kGrid) / 8u);
     const dim3 sgrid(5u * kStripes * std::min((q.cs + kBlock - 1) / kBlock, most));
     for (uint32_t it = 0; it < iterations; ++it) {

@@ -10,7 +10,7 @@
 namespace rt {
 
 // A context's work space for builds: device memory grown on demand and kept
-// for the next build (allocating and freeing ~170 B per triangle took longer
+// for the next build (allocating and freeing ~130 B per triangle took longer
 // than the kernels) up to kKeep bytes, and a pinned block for the read-backs.
 // Builds of one context run one at a time under its lock, on its stream.
 struct BvhBuildSpace {

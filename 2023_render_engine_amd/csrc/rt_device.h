@@ -359,11 +359,13 @@ __device__ __forceinline__ bool trav_step(TravState &s, const float4 *__restrict
     return true;
 }
 
-// What bounds it (16M rays, 1M triangles): the L1's address and data path is
-// busy all the time (four 16-byte loads per visit, 33 lanes of 64 active) and
-// the vector units 81 % of it.  A visit is 125 vector instructions and no
-// branch: with conversions, and branches around each push, it was 135 and ten
-// branches, and the launch took 5.03 ms instead of 4.82.
+// What bounds it (16M rays, 1M triangles, 4.85 ms): no one unit.  The vector
+// units issue 77 % of the time with 37 of 64 lanes active; the L1 takes 0.73
+// lookups per clock, as nearly every lane's 16-byte load is a lookup of its own
+// (1.96e9 for 2.12e9 loads); wavefronts wait 18 % of their life at four per
+// SIMD.  A visit is 125 vector instructions and no branch: with conversions,
+// and branches around each push, it was 135 and ten branches, 33 of 64 lanes
+// were active, and the launch took 5.03 ms.
 //
 // One step over the four-wide quantized tree (Node4, rt_internal.h): the
 // four child boxes are dequantized with one FMA per bound against the

@@ -11,8 +11,8 @@
 // sized to fill the chip; each 64-lane wavefront keeps its lanes busy by
 // refilling lanes whose ray finished (one atomic per refill per wavefront),
 // so a few long rays no longer hold 63 idle lanes hostage (incoherent rays
-// differ in visit count by an order of magnitude).  The rays are cut into
-// kStripes contiguous ranges with one claim counter each (rt_device.h), so
+// differ in visit count by an order of magnitude).  The rays are dealt to
+// kStripes stripes with one claim counter each (rt_deal.h, rt_device.h), so
 // the refills of the whole chip do not queue on one address.
 //
 // Replaces BVH::intersectRay (cuda_libraries/BVH.cu:355-448), which visits

@@ -122,7 +122,9 @@ rt_status rt_bvh_build(rt_ctx *ctx, const float *xyz, uint32_t nv, const uint32_
  * takes milliseconds instead of hundreds.  Everything rt_bvh_build's tree
  * supports works on it; export4 of a two-wide build copies nothing
  * (num_nodes4 = 0).  Invalid indices or non-finite coordinates return
- * RT_ERR_INVALID. */
+ * RT_ERR_INVALID.  The context keeps the build's work space (about 130 bytes
+ * per triangle, at most 512 MB of it) for its next build, until it is
+ * destroyed. */
 rt_status rt_bvh_build_device(rt_ctx *ctx, const float *xyz, uint32_t nv, const uint32_t *idx,
                               uint32_t nt, const rt_bvh_opts *opts, rt_bvh **out);
 rt_status rt_bvh_destroy(rt_bvh *bvh);
@@ -140,7 +142,8 @@ rt_status rt_bvh_export(const rt_bvh *bvh, float *nodes, float *tris);
 /* Copy the four-wide tree (num_nodes4 * 16 floats): per node the origin,
  * a word of scale exponents and slot-valid bits, four child links and the
  * 8-bit quantized child bounds (lo_x, hi_x, lo_y, hi_y, lo_z, hi_z words,
- * byte i = child i), followed by two zero words. */
+ * byte i = child i), followed by two zero words.  Along an axis on which the
+ * children span more than 255 * 2^50 they have no bounds: the origin is NaN. */
 rt_status rt_bvh_export4(const rt_bvh *bvh, float *nodes4);
 
 /* ------------------------------------------------------------------ */
