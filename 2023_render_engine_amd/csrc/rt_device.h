@@ -248,13 +248,12 @@ __device__ __forceinline__ int32_t stack_get(const S &st, int sp)
 }
 
 // LDS bytes of a workgroup of `block` lanes whose tree needs `stack_cap`
-// entries per lane.
+// entries per lane: its pending ones (at most stack_cap - 1) and the mark at
+// the bottom, and for the four-wide walk the place past the last entry.
 template <class S>
-inline size_t stack_lds_bytes(uint32_t stack_cap, uint32_t block)
+inline size_t stack_lds_bytes(uint32_t stack_cap, uint32_t block, bool wide = true)
 {
-    // one entry more than the four-wide walk's pending ones (stack_cap - 1 of
-    // them): the mark at the bottom and the place past the last entry
-    const uint32_t need = stack_cap + 1;
+    const uint32_t need = stack_cap + (wide ? 1u : 0u);
     const uint32_t lds = S::kTail == 0 || need < (uint32_t)S::kLds ? need : (uint32_t)S::kLds;
     return (size_t)lds * block * sizeof(int32_t);
 }
@@ -322,7 +321,7 @@ __device__ __forceinline__ bool trav_step(TravState &s, const float4 *__restrict
         const int32_t c0 = __float_as_int(d.x), c1 = __float_as_int(d.y);
         if (h0 && h1) {
             const bool swap = t1 < t0;
-            if (s.sp < cap + kStackBase) {
+            if (s.sp < cap) {
                 stack_put(stack, s.sp, swap ? c0 : c1);
                 ++s.sp;
             }

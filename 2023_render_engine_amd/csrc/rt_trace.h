@@ -34,7 +34,6 @@ struct DevBvh {
 hipError_t launch_trace(const DevBvh &bvh, const RaysDev &rays, uint32_t n, int32_t *prim, float *t,
                         uint8_t *occluded, bool any, hipStream_t stream, unsigned long long *counters,
                         uint32_t *ray_counter, bool opaque = false);
-size_t trace_lds_bytes(uint32_t stack_cap);
 // zeroes the kStripes claim counters of ray_counter (a kernel, so it can be
 // captured into a graph)
 hipError_t clear_claims(uint32_t *ray_counter, hipStream_t stream);

@@ -99,7 +99,7 @@ hipError_t launch_trace(const DevBvh &bvh, const RaysDev &rays, uint32_t n, int3
         if (e != hipSuccess || g_cus <= 0) g_cus = 256;
     }
     const int cap = (int)bvh.stack_cap;
-    const size_t lds = trace_lds_bytes(bvh.stack_cap);
+    const size_t lds = stack_lds_bytes<TraceStack>(bvh.stack_cap, kTraceBlock, bvh.wide != 0);
     // persistent launch: as many workgroups as fit (LDS-limited, at most 16
     // per CU), never more than the rays need
     size_t per_cu = lds ? (160u * 1024u) / lds : 16;
@@ -136,11 +136,6 @@ hipError_t clear_claims(uint32_t *ctr, hipStream_t stream)
 {
     hipLaunchKernelGGL(k_clear_claims, dim3(1), dim3(kStripes), 0, stream, ctr);
     return hipGetLastError();
-}
-
-size_t trace_lds_bytes(uint32_t stack_cap)
-{
-    return stack_lds_bytes<TraceStack>(stack_cap, kTraceBlock);
 }
 
 }  // namespace rt

@@ -367,7 +367,7 @@ static inline int32_t as_i32(float f) { int32_t i; memcpy(&i, &f, 4); return i; 
 static inline void kernel_inv_dir(const float d[3], float inv[3], float oinv[3], const float o[3])
 {
     for (int k = 0; k < 3; ++k) {
-        float dd = fabsf(d[k]) > 1e-30f ? d[k] : copysignf(1e-30f, d[k]);
+        float dd = fabsf(d[k]) > 1e-16f ? d[k] : copysignf(1e-16f, d[k]); /* the kernel's kMinDir */
         inv[k] = 1.0f / dd;
         oinv[k] = o[k] * inv[k];
     }

@@ -243,6 +243,11 @@ def test_traversal_stack_bound(rt, orc, gpu_ctx, n, cap):
     assert np.array_equal(prim[same], p2[same]) and np.all((prim >= steps) == (p2 >= steps))
     assert np.array_equal(occ, (p2 >= 0) & (t2 <= 10.0))
     bvh.close()
+    two = device_bvh(rt, gpu_ctx, xyz, idx, max_leaf=1, width=2)
+    t = two.trace_closest(*to_dev(rays))[1]
+    torch.cuda.synchronize()
+    assert np.array_equal(t.cpu().numpy(), t2)
+    two.close()
     # one entry more is refused
     if cap == 128:
         with pytest.raises(rt.RtError):

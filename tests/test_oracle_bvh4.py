@@ -183,3 +183,26 @@ def test_self_candidates_do_not_hide_hits(rt, orc):
     ref, _ = orc.RefBvh(d.xyz, d.idx).trace(rays)
     assert (ref[masked] < 0).sum() > 0, "the reference's order loses some of these hits"
     assert np.array_equal(ref[~masked], bp[~masked])
+
+
+def test_huge_spans_are_not_bounded(rt, orc):
+    """Children that span more than 255 * 2^50 along an axis have no bounds on
+    it (a NaN origin), so no node's scale is beyond 2^50 and slab distances stay
+    finite; the walk passes over NaN distances and finds what brute force
+    finds."""
+    xyz, idx = rt.gen_soup(300, seed=9, edge_mu=0.2)
+    xyz = np.concatenate([xyz, np.float32([[0.2, 0.3, 5.0], [0.4, 0.1, 6.0], [1e34, -2e33, 3e33]])])
+    idx = np.concatenate([idx, np.uint32([[len(xyz) - 3, len(xyz) - 2, len(xyz) - 1]])])
+    inf, nodes, nodes4, tris = host_bvh4(rt, xyz, idx)
+    meta = nodes4.copy().view(np.uint32)[:, 3]
+    scale = np.stack([(meta >> (8 * a)) & 0xFF for a in range(3)], 1).astype(int) - 127
+    assert scale.max() <= 50
+    assert np.isnan(nodes4[0, :3]).all()  # the root spans it on every axis
+    assert np.all(np.isfinite(nodes4[:, :3]) | (scale == 50))
+    rays = [a[:500].copy() for a in rt.gen_rays(1, 1, n_incoherent=500, seed=4)]
+    p4, t4, _, _, msp = orc.bvh4_trace(nodes4, tris, rays)
+    bp, bt, fl = orc.brute_trace(xyz, idx, rays)
+    clean = fl == 0
+    assert (bp[clean] >= 0).sum() > 100
+    assert np.array_equal(p4[clean], bp[clean]) and np.array_equal(t4[clean], bt[clean])
+    assert msp <= inf.stack_cap - 1
