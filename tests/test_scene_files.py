@@ -292,7 +292,8 @@ REF_OBEJOTA = ["cornellBoxGuion.obejota", "box.obejota", "models/bath/bath.obejo
                "models/kaerMorhen/kaerMorhen.obejota"]
 
 
-@pytest.mark.skipif(not os.path.isdir(REF), reason="the reference's scene files are not present")
+@pytest.mark.skipif(not os.path.isfile(os.path.join(REF, REF_OBEJOTA[0])),
+                    reason="the reference's scene files are not present")
 @pytest.mark.parametrize("name", REF_OBEJOTA)
 def test_reference_obejota_files(exe, name):
     path = os.path.join(REF, name)
@@ -309,7 +310,8 @@ def test_reference_obejota_files(exe, name):
         assert sc.lights == [((0, 0, 0.25), (1, 1, 1), 5)]
 
 
-@pytest.mark.skipif(not os.path.isdir(REF), reason="the reference's scene files are not present")
+@pytest.mark.skipif(not os.path.isfile(os.path.join(REF, REF_OBEJOTA[0])),
+                    reason="the reference's scene files are not present")
 def test_reference_mtl_files():
     m = sf.load_mtl(os.path.join(REF, "models/bath/bath.mtl"))
     illum = sorted(x.illum for x in m.values())
